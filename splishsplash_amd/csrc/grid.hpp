@@ -101,13 +101,15 @@ void build_lists_colmajor(hipStream_t s, const float4 *q, unsigned nq, const flo
                           unsigned *cnt, unsigned *maxcnt, KernelTimer &T, const char *name,
                           unsigned *nbr16 = nullptr, unsigned *ovf16 = nullptr);
 
-// CSR variant for the drop-in search: queries in caller order, sources
-// cell-sorted with srcmap[slot] = caller index of the source point. With
-// rowoff == nullptr only counts are written (pass 1); with rowoff the lists
-// are written at out[rowoff[i] ...] (pass 2). same_set excludes
-// srcmap[slot] == i.
-void build_lists_csr(hipStream_t s, const float4 *q, unsigned nq, const float4 *src, const unsigned *srcmap,
-                     const unsigned *start, const GridDesc &g, float r2, bool same_set, const unsigned *rowoff,
-                     unsigned *out, unsigned *cnt);
+// CSR variant for the drop-in search: sources cell-sorted with srcmap[slot] =
+// caller index of the source point, queries q with qmap[k] = caller index of
+// query k (null: k itself), best in cell order too. With rowoff == nullptr
+// only counts are written (pass 1, cnt[caller index]); with rowoff the lists
+// are written at out[rowoff[caller index] ...] (pass 2), row by row and in
+// slot order, whatever the order of the queries. same_set: q is the source
+// array itself (query k in slot k), and a point is not its own neighbour.
+void build_lists_csr(hipStream_t s, const float4 *q, const unsigned *qmap, unsigned nq, const float4 *src,
+                     unsigned nsrc, const unsigned *srcmap, const unsigned *start, const GridDesc &g, double radius, bool same_set,
+                     const unsigned *rowoff, unsigned *out, unsigned *cnt);
 
 }  // namespace sph

@@ -186,8 +186,7 @@ extern "C" int sph_ns_find_neighbors_noalloc(const float *x, size_t n, double ra
         const CellSortBufs b{start, pcell, perm, keys2, vals2, hist, hoff, bsum};
         cell_sort_raw(s, x4, nn, g, b, T);
         permute_f4(s, perm, nn, x4, srt);
-        const float r2 = (float)radius * (float)radius;
-        build_lists_csr(s, x4, nn, srt, perm, start, g, r2, true, nullptr, nullptr, cnt);
+        build_lists_csr(s, srt, perm, nn, srt, nn, perm, start, g, radius, true, nullptr, nullptr, cnt);
         exclusive_scan_raw(s, cnt, offsets, nn, bsum, T);
         unsigned tot = 0;
         SPH_HIP(hipMemcpyAsync(&tot, offsets + n, sizeof(unsigned), hipMemcpyDeviceToHost, s));
@@ -197,7 +196,7 @@ extern "C" int sph_ns_find_neighbors_noalloc(const float *x, size_t n, double ra
                     "sph_ns_find_neighbors_noalloc: " + std::to_string(tot) + " neighbour entries exceed the capacity of " +
                         std::to_string(capacity) + " (offsets are written; *total holds the size needed)");
         SPH_REQUIRE(neighbors || tot == 0, SPH_ERR_INVALID, "sph_ns_find_neighbors_noalloc: null neighbour buffer");
-        if (tot) build_lists_csr(s, x4, nn, srt, perm, start, g, r2, true, offsets, neighbors, nullptr);
+        if (tot) build_lists_csr(s, srt, perm, nn, srt, nn, perm, start, g, radius, true, offsets, neighbors, nullptr);
         SPH_HIP(hipStreamSynchronize(s));
     });
 }

@@ -83,7 +83,6 @@ static void find(NSHandle &h, bool points_changed) {
     if (!any)
         for (int c = 0; c < 3; c++) lo[c] = hi[c] = 0.0;
     const GridDesc g = make_grid(lo, hi, h.radius);
-    const float r2 = (float)h.radius * (float)h.radius;
     // sort every set that some set searches in
     std::vector<bool> needed(ns, false);
     for (size_t i = 0; i < ns; i++)
@@ -106,8 +105,11 @@ static void find(NSHandle &h, bool points_changed) {
             if (!h.active[i][j] || qi.n == 0 || h.sets[j]->n == 0) continue;
             PointSet &sj = *h.sets[j];
             cnt.reserve(qi.n);
-            build_lists_csr(h.stream, qi.dx.get(), (unsigned)qi.n, sj.dsorted.get(), sj.sorter.perm.get(),
-                            sj.sorter.start.get(), g, r2, i == j, nullptr, nullptr, cnt.get());
+            // queries in cell order where the set has been sorted
+            const float4 *q = needed[i] ? qi.dsorted.get() : qi.dx.get();
+            const unsigned *qmap = needed[i] ? qi.sorter.perm.get() : nullptr;
+            build_lists_csr(h.stream, q, qmap, (unsigned)qi.n, sj.dsorted.get(), (unsigned)sj.n,
+                            sj.sorter.perm.get(), sj.sorter.start.get(), g, h.radius, i == j, nullptr, nullptr, cnt.get());
             off.reserve(qi.n + 1);
             exclusive_scan(h.stream, cnt.get(), off.get(), (unsigned)qi.n, qi.sorter.bsum, h.timer);
             SPH_HIP(hipMemcpyAsync(qi.off[j].data(), off.get(), (qi.n + 1) * sizeof(unsigned), hipMemcpyDeviceToHost,
@@ -117,8 +119,8 @@ static void find(NSHandle &h, bool points_changed) {
             qi.idx[j].resize(total);
             if (!total) continue;
             out.reserve(total);
-            build_lists_csr(h.stream, qi.dx.get(), (unsigned)qi.n, sj.dsorted.get(), sj.sorter.perm.get(),
-                            sj.sorter.start.get(), g, r2, i == j, off.get(), out.get(), nullptr);
+            build_lists_csr(h.stream, q, qmap, (unsigned)qi.n, sj.dsorted.get(), (unsigned)sj.n,
+                            sj.sorter.perm.get(), sj.sorter.start.get(), g, h.radius, i == j, off.get(), out.get(), nullptr);
             SPH_HIP(hipMemcpyAsync(qi.idx[j].data(), out.get(), total * sizeof(unsigned), hipMemcpyDeviceToHost,
                                    h.stream));
             SPH_HIP(hipStreamSynchronize(h.stream));

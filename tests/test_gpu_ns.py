@@ -199,3 +199,54 @@ def test_empty_and_tiny_sets():
     assert ns.point_set(b).n_neighbors(b, 0) == 0
     assert ns.point_set(b).n_neighbors(a, 0) == 0
     assert ns.point_set(a).n_points() == 0
+
+
+def expected_csr(x, radius, y=None):
+    """The drop-in search's lists in its own order: (dz, dy) row, then cell
+    along x, then point index (FP32 cell coordinates and inclusion test)."""
+    src = x if y is None else y
+    lo = np.minimum(x.min(0), src.min(0)).astype(np.float64)
+    cs = radius * (1.0 + 1e-4)
+    o, inv = (lo - cs).astype(np.float32), np.float32(1.0 / cs)
+    cell = lambda p: np.floor((p - o) * inv).astype(np.int64)
+    off, idx = oracle.neighbors(x, y, radius=np.float32(radius))
+    i = np.repeat(np.arange(len(x)), np.diff(off.astype(np.int64)))
+    d = cell(src)[idx] - cell(x)[i]
+    order = np.lexsort((idx, d[:, 0], d[:, 1], d[:, 2], i))
+    return off, idx[order]
+
+
+@pytest.mark.parametrize("n,knot", [(1, 0), (63, 0), (65, 40), (700, 700), (5003, 900), (131071, 0), (131072, 0),
+                                    (131109, 1500)])
+def test_drop_in_lists_keep_their_order(n, knot):
+    """Sizes around a wave and around the switch between a wave and a lane
+    per query; `knot` points crowd into a corner of one cell, so that rows
+    hold far more candidates than one window or hit word."""
+    rng = np.random.default_rng(n)
+    x = rng.uniform(0.0, 1.0, (n, 3)).astype(np.float32)
+    r = max(radius_for(n, 20.0), 0.02) if n > 1 else 0.1
+    x[rng.permutation(n)[:knot]] = (0.5 + rng.uniform(0.0, 0.6 * r, (knot, 3))).astype(np.float32)
+    ns = capi.NeighborhoodSearch(r)
+    i = ns.add_point_set(x)
+    ns.find_neighbors()
+    off, idx = ns.neighbors_csr(i, i)
+    off_e, idx_e = expected_csr(x, r)
+    np.testing.assert_array_equal(off, off_e)
+    np.testing.assert_array_equal(idx, idx_e)
+
+
+@pytest.mark.parametrize("n", [300, 140007])
+def test_drop_in_lists_of_two_sets_keep_their_order(n):
+    rng = np.random.default_rng(n)
+    x = rng.uniform(0.0, 1.0, (n, 3)).astype(np.float32)
+    y = scenes.box_wall_particles((-0.1, 0, 0), (1, 1, 1), 0.05).astype(np.float32)
+    r = 0.06
+    ns = capi.NeighborhoodSearch(r)
+    # the queries' own set is not searched, so it is not in cell order
+    a = ns.add_point_set(x, True, True, False)
+    b = ns.add_point_set(y, False, False, True)
+    ns.find_neighbors()
+    off, idx = ns.neighbors_csr(a, b)
+    off_e, idx_e = expected_csr(x, r, y)
+    np.testing.assert_array_equal(off, off_e)
+    np.testing.assert_array_equal(idx, idx_e)

@@ -114,3 +114,30 @@ def test_noalloc_capacity_and_limits():
     rc = capi.lib().sph_ns_find_neighbors_noalloc(None, (1 << 19) + 1, radius, None, None, 0, C.byref(total), None)
     assert rc == SPH_ERR_RANGE
     assert "maximum" in capi.lib().sph_last_error().decode()
+
+
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_lists_at_any_output_alignment(shift):
+    """Large sets are written in groups of four entries: the lists are whole
+    and the words around them untouched at every alignment of the buffer."""
+    n, radius = 131_200, 0.025
+    x = np.random.default_rng(5).random((n, 3)).astype(np.float32)
+    off_r, idx_r = drop_in(x, radius)
+    hip = Hip()
+    pad = 8
+    xd, od, nd = hip.alloc(12 * n), hip.alloc(4 * (n + 1)), hip.alloc(4 * (len(idx_r) + 2 * pad))
+    try:
+        hip.put(xd, x.reshape(-1))
+        hip.put(nd, np.full(len(idx_r) + 2 * pad, 0xABCDEF01, np.uint32))
+        total = C.c_size_t(0)
+        rc = capi.lib().sph_ns_find_neighbors_noalloc(xd, n, radius, od, C.c_void_p(nd.value + 4 * (pad - shift)),
+                                                      len(idx_r), C.byref(total), None)
+        off = hip.get(od, np.zeros(n + 1, np.uint32))
+        buf = hip.get(nd, np.zeros(len(idx_r) + 2 * pad, np.uint32))
+    finally:
+        hip.free(xd, od, nd)
+    assert rc == 0 and total.value == len(idx_r)
+    np.testing.assert_array_equal(off, off_r)
+    lo = pad - shift
+    np.testing.assert_array_equal(buf[lo:lo + len(idx_r)], idx_r)
+    assert (buf[:lo] == 0xABCDEF01).all() and (buf[lo + len(idx_r):] == 0xABCDEF01).all()

@@ -56,43 +56,296 @@ __global__ void k_reset(Ctl *C, int which) {
 // TimeStep::computeDensities (TimeStep.cpp:116-169), computeDFSPHFactor
 // (TimeStepDFSPH.cpp:1106-1186), computeDensityChange + divergence warm start
 // (TimeStepDFSPH.cpp:398-463, 1247-1295).
-// The fluid neighbours of particle i taken by lane hl of the particle's LPP
-// lanes: g4(j0, j1, j2, j3) for groups of four (all four indices loaded
-// before the call, so the caller can issue their gathers together) and
-// g1(j) for the rest. From the packed lists lane hl takes words hl,
-// hl + LPP, ... (two neighbours each); from nf neighbours hl, hl + LPP, ....
-// The split is fixed by (cnt, LPP, which list), so sums stay deterministic.
 __device__ __forceinline__ unsigned nb_lo(unsigned i, unsigned w) { return i + (unsigned)(int)(short)(w & 0xffffu); }
 __device__ __forceinline__ unsigned nb_hi(unsigned i, unsigned w) { return i + (unsigned)((int)w >> 16); }
 
-template <int LPP, class G4, class G1>
-__device__ __forceinline__ void fluid_nbrs4(const Dev &D, unsigned i, unsigned hl, unsigned cnt, G4 &&g4, G1 &&g1) {
+// What a sweep loads per neighbour: up to three arrays (a, b, c of the
+// result). Groups of neighbours are loaded array by array: the gathers of
+// one array together measured 2-5 % faster than neighbour by neighbour
+// (k_jacobi, k_jacobi2, k_features at 1M particles).
+struct NoLoad {
+    __device__ int operator()(unsigned) const { return 0; }
+};
+template <class A, class B, class C> struct Neighbour {
+    A a;
+    B b;
+    C c;
+};
+template <class A, class B, class C> struct Loads {
+    A a;
+    B b;
+    C c;
+    __device__ __forceinline__ auto operator()(unsigned j) const {
+        return Neighbour<decltype(a(j)), decltype(b(j)), decltype(c(j))>{a(j), b(j), c(j)};
+    }
+    // q[k] = the neighbour j[k], k < 4
+    template <class Q> __device__ __forceinline__ void four(const unsigned *j, Q *q) const {
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k].a = a(j[k]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k].b = b(j[k]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k].c = c(j[k]);
+    }
+};
+template <class A, class B = NoLoad, class C = NoLoad>
+__device__ __forceinline__ Loads<A, B, C> loads(A a, B b = B{}, C c = C{}) {
+    return {a, b, c};
+}
+
+// Calls f(j, ld(j)) for the fluid neighbours of particle i taken by lane hl
+// of the particle's LPP lanes, the loads of four neighbours issued before
+// the first f. From the packed lists lane hl takes words hl, hl + LPP, ...
+// (two neighbours each); from nf neighbours hl, hl + LPP, .... The split is
+// fixed by (cnt, LPP, which list), so sums stay deterministic.
+template <int LPP, class LD, class F>
+__device__ __forceinline__ void fluid_pairs(const Dev &D, unsigned i, unsigned hl, unsigned cnt, LD &&ld, F &&f) {
     const size_t S = D.stride;
+    auto four = [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
+        const unsigned j[4] = {j0, j1, j2, j3};
+        decltype(ld(0u)) q[4];
+        ld.four(j, q);
+        f(j0, q[0]);
+        f(j1, q[1]);
+        f(j2, q[2]);
+        f(j3, q[3]);
+    };
     if (D.nf16) {
         const unsigned *__restrict__ P = D.nf16 + i;
         const unsigned full = cnt >> 1;  // words holding two neighbours
         unsigned w = hl;
         for (; w + LPP < full; w += 2 * LPP) {
             const unsigned a = P[w * S], b = P[(w + LPP) * S];
-            g4(nb_lo(i, a), nb_hi(i, a), nb_lo(i, b), nb_hi(i, b));
+            four(nb_lo(i, a), nb_hi(i, a), nb_lo(i, b), nb_hi(i, b));
         }
         for (; w < full; w += LPP) {
             const unsigned a = P[w * S];
-            g1(nb_lo(i, a));
-            g1(nb_hi(i, a));
+            f(nb_lo(i, a), ld(nb_lo(i, a)));
+            f(nb_hi(i, a), ld(nb_hi(i, a)));
         }
-        if ((cnt & 1u) && w == full) g1(nb_lo(i, P[w * S]));
+        if ((cnt & 1u) && w == full) {
+            const unsigned j = nb_lo(i, P[w * S]);
+            f(j, ld(j));
+        }
     } else {
         const unsigned *__restrict__ L = D.nf + i;
         unsigned k = hl;
         for (; k + 3 * LPP < cnt; k += 4 * LPP)
-            g4(L[k * S], L[(k + LPP) * S], L[(k + 2 * LPP) * S], L[(k + 3 * LPP) * S]);
-        for (; k < cnt; k += LPP) g1(L[k * S]);
+            four(L[k * S], L[(k + LPP) * S], L[(k + 2 * LPP) * S], L[(k + 3 * LPP) * S]);
+        for (; k < cnt; k += LPP) f(L[k * S], ld(L[k * S]));
     }
 }
 
+// Calls f(xb) for the Akinci boundary neighbours of particle i in order.
+template <class F>
+__device__ __forceinline__ void akinci_pairs(const Dev &D, unsigned i, unsigned cb, F &&f) {
+    for (unsigned k = 0; k < cb; k++) f(D.bx[D.nb[(size_t)k * D.stride + i]]);
+}
+// Neighbour sums may be split over LPP = 2 or 4 adjacent lanes: lane h of a
+// particle takes words (or neighbours) h, h + LPP, ..., and the partial sums
+// are combined by butterfly shuffles in a fixed order (results are
+// deterministic; LPP = 1 is the plain sequential sum). Shorter per-lane
+// chains of dependent gathers keep more loads in flight per wave.
 template <int LPP>
-__device__ __forceinline__ float lane_sum(float v);
+__device__ __forceinline__ float lane_sum(float v) {
+    if (LPP >= 2) v += __shfl_xor(v, 1, 64);
+    if (LPP >= 4) v += __shfl_xor(v, 2, 64);
+    return v;
+}
+
+// LPP = ORDERED_LANES shares a particle's pairs over 16 lanes without
+// changing the sum: the lanes evaluate up to 64 pairs at once (all their
+// index loads, then all their gathers in flight), leave the terms in LDS, and
+// one lane per accumulator then adds them in list order, exactly as one lane
+// per particle would. For counts that leave the GPU mostly idle: a sweep
+// there takes as long as its chain of dependent loads, which this cuts from
+// about one per four neighbours to two, and the ordered adds from LDS take a
+// few hundred cycles.
+constexpr int ORDERED_LANES = 16;
+constexpr int ORDERED_SLOTS = 64;
+
+// What a sweep sums per pair: NT terms t and NACC accumulators,
+// acc[c] = fma(t[a(c)], t[b(c)], acc[c]), or acc[c] += t[c] with ADD.
+template <int N> struct SumAdd {
+    static constexpr int NT = N, NACC = N;
+    static constexpr bool ADD = true;
+    static constexpr int a(int c) { return c; }
+    static constexpr int b(int) { return 0; }
+};
+struct SumVec {  // t = (c, x, y, z): acc += c (x, y, z)
+    static constexpr int NT = 4, NACC = 3;
+    static constexpr bool ADD = false;
+    static constexpr int a(int) { return 0; }
+    static constexpr int b(int c) { return 1 + c; }
+};
+struct SumDot {  // t = (g, d): acc += g d
+    static constexpr int NT = 2, NACC = 1;
+    static constexpr bool ADD = false;
+    static constexpr int a(int) { return 0; }
+    static constexpr int b(int) { return 1; }
+};
+struct SumSym {  // t = (u, r): acc += the upper triangle of u r^T
+    static constexpr int NT = 6, NACC = 6;
+    static constexpr bool ADD = false;
+    static constexpr int a(int c) { return c < 3 ? 0 : (c < 5 ? 1 : 2); }
+    static constexpr int b(int c) { return c < 3 ? 3 + c : (c < 5 ? 1 + c : 5); }
+};
+struct SumVecAdd {  // t = (x, y, z | c, u, v, w): acc += (x, y, z), c (u, v, w)
+    static constexpr int NT = 8, NACC = 6;  // t[7] = 1
+    static constexpr bool ADD = false;
+    static constexpr int a(int c) { return c < 3 ? c : 3; }
+    static constexpr int b(int c) { return c < 3 ? 7 : 1 + c; }
+};
+
+template <class S> __device__ __forceinline__ void sum_terms(const float *t, float *acc) {
+#pragma unroll
+    for (int c = 0; c < S::NACC; c++)
+        acc[c] = S::ADD ? acc[c] + t[c] : fmaf(t[S::a(c)], t[S::b(c)], acc[c]);
+}
+
+// Floats of LDS per particle for up to NT terms per pair (a multiple of four
+// off the banks' period, so the four particles of a wave read different
+// banks), per block, and a particle's own part. Every sum of a kernel uses
+// the same part: the waves of a block are not in step.
+template <int NT> constexpr int PAIR_PITCH = ORDERED_SLOTS * NT + 4;
+template <int LPP, int NT>
+constexpr int PAIR_LDS = LPP == ORDERED_LANES ? (BLOCK / ORDERED_LANES) * PAIR_PITCH<NT> : 1;
+template <int LPP, int NT> __device__ __forceinline__ float *pair_part(float *lds) {
+    return LPP == ORDERED_LANES ? lds + (threadIdx.x / ORDERED_LANES) * PAIR_PITCH<NT> : nullptr;
+}
+
+// A particle's LDS accesses stay within its wave, which executes them in
+// program order: only the compiler must keep that order.
+__device__ __forceinline__ void pair_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Adds the terms of slots 0 .. m - 1 in order; lane c < NACC of the particle
+// holds accumulator c, in and out.
+template <class S>
+__device__ __forceinline__ void ordered_add(const float *__restrict__ T, unsigned hl, unsigned m, float &my) {
+    pair_sync();
+    if (hl < (unsigned)S::NACC) {
+        int oa = 0, ob = 0;
+#pragma unroll
+        for (int c = 0; c < S::NACC; c++)
+            if (hl == (unsigned)c) {
+                oa = S::a(c);
+                ob = S::b(c);
+            }
+#pragma unroll 8
+        for (unsigned k = 0; k < m; k++)
+            my = S::ADD ? my + T[k * S::NT + oa] : fmaf(T[k * S::NT + oa], T[k * S::NT + ob], my);
+    }
+    pair_sync();
+}
+template <class S, class V> __device__ __forceinline__ void ordered_put(float *__restrict__ T, unsigned slot, V &&term) {
+    float t[S::NT];
+    if (!term(t))
+#pragma unroll
+        for (int q = 0; q < S::NT; q++) t[q] = 0.f;
+#pragma unroll
+    for (int q = 0; q < S::NT; q++) T[slot * S::NT + q] = t[q];
+}
+template <class S> __device__ __forceinline__ float ordered_mine(unsigned hl, const float *acc) {
+    float my = 0.f;
+#pragma unroll
+    for (int c = 0; c < S::NACC; c++)
+        if (hl == (unsigned)c) my = acc[c];
+    return my;
+}
+template <class S> __device__ __forceinline__ void ordered_share(float my, float *acc) {
+#pragma unroll
+    for (int c = 0; c < S::NACC; c++) acc[c] = __shfl(my, c, ORDERED_LANES);
+}
+
+// Sums over the cnt fluid neighbours of particle i: ld(j) loads a
+// neighbour's data, term(j, data, t) writes its terms and returns whether
+// they count; T is the particle's part of LDS. Every lane of the particle
+// calls this; acc is the starting value and, after lanes_join, the result in
+// each lane of it.
+template <int LPP, class S, class LD, class TERM>
+__device__ __forceinline__ void fluid_sums(const Dev &D, unsigned i, unsigned hl, unsigned cnt, float *__restrict__ T,
+                                           float *acc, LD &&ld, TERM &&term) {
+    if constexpr (LPP != ORDERED_LANES) {
+        fluid_pairs<LPP>(D, i, hl, cnt, ld, [&](unsigned j, const auto &q) {
+            float t[S::NT];
+            if (term(j, q, t)) sum_terms<S>(t, acc);
+        });
+    } else {
+        float my = ordered_mine<S>(hl, acc);
+        const size_t N = D.stride;
+        for (unsigned k0 = 0; k0 < cnt; k0 += ORDERED_SLOTS) {
+            // slots of this lane: 2 hl, 2 hl + 1 (one packed word) and the
+            // same in the second half; the missing ones read slot 0's
+            // neighbour
+            unsigned j[4], sl[4];
+#pragma unroll
+            for (unsigned u = 0; u < 2; u++) {
+                sl[2 * u] = 32 * u + 2 * hl;
+                sl[2 * u + 1] = sl[2 * u] + 1;
+                const unsigned a = k0 + sl[2 * u], b = a + 1;
+                if (D.nf16) {
+                    const unsigned w = D.nf16[(size_t)((a < cnt ? a : k0) >> 1) * N + i];
+                    j[2 * u] = nb_lo(i, w);
+                    j[2 * u + 1] = nb_hi(i, w);
+                } else {
+                    j[2 * u] = D.nf[(size_t)(a < cnt ? a : k0) * N + i];
+                    j[2 * u + 1] = D.nf[(size_t)(b < cnt ? b : k0) * N + i];
+                }
+            }
+            decltype(ld(0u)) q[4];
+            ld.four(j, q);
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++)
+                if (k0 + sl[u] < cnt) ordered_put<S>(T, sl[u], [&](float *t) { return term(j[u], q[u], t); });
+            ordered_add<S>(T, hl, cnt - k0 < ORDERED_SLOTS ? cnt - k0 : ORDERED_SLOTS, my);
+        }
+        ordered_share<S>(my, acc);
+    }
+}
+
+// Combines the lanes' sums; every lane of the wave calls this.
+template <int LPP, class S> __device__ __forceinline__ void lanes_join(float *acc) {
+    if (LPP > 1 && LPP != ORDERED_LANES)
+#pragma unroll
+        for (int c = 0; c < S::NACC; c++) acc[c] = lane_sum<LPP>(acc[c]);
+}
+
+// The same over the Akinci boundary neighbours (cb of them), in list order
+// by one lane of the particle (acc valid in lane hl == 0), or shared as
+// above.
+template <int LPP, class S, class TERM>
+__device__ __forceinline__ void akinci_sums(const Dev &D, unsigned i, unsigned hl, unsigned cb,
+                                            float *__restrict__ T, float *acc, TERM &&term) {
+    if constexpr (LPP != ORDERED_LANES) {
+        if (hl == 0)
+            akinci_pairs(D, i, cb, [&](const float4 &xb) {
+                float t[S::NT];
+                if (term(xb, t)) sum_terms<S>(t, acc);
+            });
+    } else {
+        float my = ordered_mine<S>(hl, acc);
+        for (unsigned k0 = 0; k0 < cb; k0 += ORDERED_SLOTS) {
+            unsigned j[4];
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++) {
+                const unsigned k = k0 + 16 * u + hl;
+                j[u] = D.nb[(size_t)(k < cb ? k : k0) * D.stride + i];
+            }
+            float4 q[4];
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++) q[u] = D.bx[j[u]];
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++)
+                if (k0 + 16 * u + hl < cb) ordered_put<S>(T, 16 * u + hl, [&](float *t) { return term(q[u], t); });
+            ordered_add<S>(T, hl, cb - k0 < ORDERED_SLOTS ? cb - k0 : ORDERED_SLOTS, my);
+        }
+        ordered_share<S>(my, acc);
+    }
+}
 
 // ParticleState::Active (FluidModel.h:75) unless the state array says
 // otherwise; without states every particle is active.
@@ -117,77 +370,97 @@ __device__ __forceinline__ float xsphB_of(const Dev &D, unsigned i) { return D.m
 
 template <bool DENS, bool FACT, bool DIV, int LPP>
 __global__ __launch_bounds__(BLOCK) void k_sweep_init(Dev D) {
+    constexpr int NF = (DENS ? 1 : 0) + (FACT ? 4 : 0) + (DIV ? 1 : 0);
+    constexpr int NB = (DENS ? 1 : 0) + (FACT ? 3 : 0) + (DIV ? 1 : 0);
+    __shared__ float plds[PAIR_LDS<LPP, NF>];
+    float *const T = pair_part<LPP, NF>(plds);
     const unsigned t = gtid();
     const unsigned i = t / LPP, hl = t % LPP;
     const bool act = i < D.n;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), vi = xi;
-    float dens = (LPP == 1) ? D.V * D.K.W0 : 0.f;
-    float sgk = 0.f, gpx = 0.f, gpy = 0.f, gpz = 0.f, div = 0.f, divb = 0.f;
-    unsigned cnt = 0;
+    unsigned cnt = 0, cb = 0;
+    // the density's own share opens the sequential sum; split sums add it
+    // to their total
+    float f[NF];
+#pragma unroll
+    for (int q = 0; q < NF; q++) f[q] = 0.f;
+    if (DENS && (LPP == 1 || LPP == ORDERED_LANES)) f[0] = D.V * D.K.W0;
     if (act) {
         xi = D.x[i];
         if (DIV) vi = D.v[i];
         cnt = D.cf[i];
-        auto pair = [&](const float4 &xj, const float4 &vj) {
-            float3 r;
-            float w, g;
-            kernel_WG(xi, xj, D.K, r, w, g);
-            if (DENS) dens += D.V * w;
-            const float gx = g * r.x, gy = g * r.y, gz = g * r.z;
-            if (FACT) {
-                const float qx = -D.V * gx, qy = -D.V * gy, qz = -D.V * gz;
-                sgk += sqn(qx, qy, qz);
-                gpx -= qx;
-                gpy -= qy;
-                gpz -= qz;
-            }
-            if (DIV) div += ((vi.x - vj.x) * gx + (vi.y - vj.y) * gy) + (vi.z - vj.z) * gz;
-        };
         const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
         const F4Gather X(D.x, D.n), V(D.v, D.n);
-        fluid_nbrs4<LPP>(
-            D, i, hl, cnt,
-            [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-                const float4 x0 = X.xyz(j0), x1 = X.xyz(j1), x2 = X.xyz(j2), x3 = X.xyz(j3);
-                const float4 v0 = DIV ? V.xyz(j0) : z4, v1 = DIV ? V.xyz(j1) : z4, v2 = DIV ? V.xyz(j2) : z4,
-                             v3 = DIV ? V.xyz(j3) : z4;
-                pair(x0, v0);
-                pair(x1, v1);
-                pair(x2, v2);
-                pair(x3, v3);
-            },
-            [&](unsigned j) { pair(X.xyz(j), DIV ? V.xyz(j) : z4); });
+        fluid_sums<LPP, SumAdd<NF>>(
+            D, i, hl, cnt, T, f, loads([&](unsigned j) { return X.xyz(j); }, [&](unsigned j) { return DIV ? V.xyz(j) : z4; }),
+            [&](unsigned, const auto &p, float *u) {
+                const float4 &vj = p.b;
+                float3 r;
+                float w, g;
+                kernel_WG(xi, p.a, D.K, r, w, g);
+                int q = 0;
+                if (DENS) u[q++] = D.V * w;
+                const float gx = g * r.x, gy = g * r.y, gz = g * r.z;
+                if (FACT) {
+                    const float qx = -D.V * gx, qy = -D.V * gy, qz = -D.V * gz;
+                    u[q++] = sqn(qx, qy, qz);
+                    u[q++] = -qx;
+                    u[q++] = -qy;
+                    u[q++] = -qz;
+                }
+                if (DIV) u[q++] = ((vi.x - vj.x) * gx + (vi.y - vj.y) * gy) + (vi.z - vj.z) * gz;
+                return true;
+            });
     }
-    if (LPP > 1) {
-        if (DENS) dens = D.V * D.K.W0 + lane_sum<LPP>(dens);
-        if (FACT) {
-            sgk = lane_sum<LPP>(sgk);
-            gpx = lane_sum<LPP>(gpx);
-            gpy = lane_sum<LPP>(gpy);
-            gpz = lane_sum<LPP>(gpz);
-        }
-        if (DIV) div = lane_sum<LPP>(div);
+    lanes_join<LPP, SumAdd<NF>>(f);
+    if (act && D.bmode == 1) cb = D.cb[i];
+    float dens = 0.f, sgk = 0.f, gpx = 0.f, gpy = 0.f, gpz = 0.f, div = 0.f, divb = 0.f;
+    if (DENS) dens = (LPP == 1 || LPP == ORDERED_LANES) ? f[0] : D.V * D.K.W0 + f[0];
+    if (FACT) {
+        constexpr int q = DENS ? 1 : 0;
+        sgk = f[q];
+        gpx = f[q + 1];
+        gpy = f[q + 2];
+        gpz = f[q + 3];
     }
-    if (!act || hl != 0) return;
-    unsigned nnb = cnt;
+    if (DIV) div = f[NF - 1];
     if (D.bmode == 1) {
-        const unsigned cb = D.cb[i];
-        nnb += cb;
-        for (unsigned k = 0; k < cb; k++) {
-            const float4 xb = D.bx[D.nb[(size_t)k * D.stride + i]];
+        float b[NB];
+        int q = 0;
+        if (DENS) b[q++] = dens;
+        if (FACT) {
+            b[q++] = gpx;
+            b[q++] = gpy;
+            b[q++] = gpz;
+        }
+        if (DIV) b[q++] = 0.f;
+        akinci_sums<LPP, SumAdd<NB>>(D, i, hl, cb, T, b, [&](const float4 &xb, float *u) {
             float3 r;
             float w, g;
             kernel_WG(xi, xb, D.K, r, w, g);
-            if (DENS) dens += xb.w * w;
+            int q = 0;
+            if (DENS) u[q++] = xb.w * w;
             const float gx = g * r.x, gy = g * r.y, gz = g * r.z;
             if (FACT) {
-                gpx -= -xb.w * gx;
-                gpy -= -xb.w * gy;
-                gpz -= -xb.w * gz;
+                u[q++] = xb.w * gx;
+                u[q++] = xb.w * gy;
+                u[q++] = xb.w * gz;
             }
-            if (DIV) divb += xb.w * (((vi.x * gx + vi.y * gy) + vi.z * gz));
+            if (DIV) u[q++] = xb.w * ((vi.x * gx + vi.y * gy) + vi.z * gz);
+            return true;
+        });
+        q = 0;
+        if (DENS) dens = b[q++];
+        if (FACT) {
+            gpx = b[q++];
+            gpy = b[q++];
+            gpz = b[q++];
         }
-    } else if (D.bmode == 2) {
+        if (DIV) divb = b[q++];
+    }
+    if (!act || hl != 0) return;
+    const unsigned nnb = cnt + cb;
+    if (D.bmode == 2) {
         for (unsigned o = 0; o < D.nvm; o++) {
             const float4 xb = D.vmb[(size_t)o * D.stride + i];
             if (!(xb.w > 0.f)) break;
@@ -259,34 +532,26 @@ __global__ __launch_bounds__(BLOCK) void k_sweep_init(Dev D) {
 // stiffness (p / rho^2 or p_v / rho^2, kept equal to the stiffness array by
 // k_stiff_to_w and the Jacobi update), so one 16-byte load per neighbour
 // gives both the position and the stiffness.
-__device__ __forceinline__ void accel_pair(const Dev &D, const float4 &xi, float pi, const float4 &xj, float &ax,
-                                           float &ay, float &az, float inv_rho0i = 1.f) {
+// t = (c, r) with a_i += c r; false where the pair carries no pressure.
+__device__ __forceinline__ bool accel_term(const Dev &D, const float4 &xi, float pi, const float4 &xj, float inv_rho0i,
+                                           float *t) {
     const float ps = D.model ? pi + xj.w * inv_rho0i : pi + xj.w;
-    if (fabsf(ps) > D.eps) {
-        float3 r;
-        const float g = kernel_G(xi, xj, D.K, r);
-        const float c = ps * (-D.V * g);  // a_i += -V (p_i + p_j) gradW_ij
-        ax = fmaf(c, r.x, ax);
-        ay = fmaf(c, r.y, ay);
-        az = fmaf(c, r.z, az);
-    }
+    if (!(fabsf(ps) > D.eps)) return false;
+    float3 r;
+    const float g = kernel_G(xi, xj, D.K, r);
+    t[0] = ps * (-D.V * g);  // a_i += -V (p_i + p_j) gradW_ij
+    t[1] = r.x;
+    t[2] = r.y;
+    t[3] = r.z;
+    return true;
 }
 
-// Boundary part of computePressureAccel for particle i (TimeStepDFSPH.cpp:1330-1365).
-__device__ __forceinline__ void accel_boundary(const Dev &D, unsigned i, const float4 &xi, float pi, float3 &acc) {
+// Map records of computePressureAccel for particle i (TimeStepDFSPH.cpp:
+// 1330-1365).
+__device__ __forceinline__ void accel_maps(const Dev &D, unsigned i, const float4 &xi, float pi, float3 &acc) {
     float ax = acc.x, ay = acc.y, az = acc.z;
     if (fabsf(pi) > D.eps) {
-        if (D.bmode == 1) {
-            const unsigned cb = D.cb[i];
-            for (unsigned k = 0; k < cb; k++) {
-                const float4 xb = D.bx[D.nb[(size_t)k * D.stride + i]];
-                float3 r;
-                const float g = kernel_G(xi, xb, D.K, r);
-                ax += pi * (-xb.w * (g * r.x));
-                ay += pi * (-xb.w * (g * r.y));
-                az += pi * (-xb.w * (g * r.z));
-            }
-        } else if (D.bmode == 2) {
+        if (D.bmode == 2) {
             for (unsigned o = 0; o < D.nvm; o++) {
                 const float4 xb = D.vmb[(size_t)o * D.stride + i];
                 if (!(xb.w > 0.f)) break;
@@ -309,77 +574,37 @@ __device__ __forceinline__ void accel_boundary(const Dev &D, unsigned i, const f
     acc = make_float3(ax, ay, az);
 }
 
-__device__ __forceinline__ float3 accel_i(const Dev &D, unsigned i, const float *__restrict__ P) {
-    const float4 xi = D.x[i];
-    const float pi = P[i];
-    const float ir = D.model ? 1.0f / rho0_of(D, i) : 1.f;
-    const F4Gather X(D.x, D.n);
-    float ax = 0.f, ay = 0.f, az = 0.f;
-    // four neighbours per trip: the index and position loads of all four are
-    // issued before the first use, so each wave keeps more gathers in flight
-    fluid_nbrs4<1>(
-        D, i, 0, D.cf[i],
-        [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-            const float4 x0 = X.all(j0), x1 = X.all(j1), x2 = X.all(j2), x3 = X.all(j3);
-            accel_pair(D, xi, pi, x0, ax, ay, az, ir);
-            accel_pair(D, xi, pi, x1, ax, ay, az, ir);
-            accel_pair(D, xi, pi, x2, ax, ay, az, ir);
-            accel_pair(D, xi, pi, x3, ax, ay, az, ir);
-        },
-        [&](unsigned j) { accel_pair(D, xi, pi, X.all(j), ax, ay, az, ir); });
-    float3 a = make_float3(ax, ay, az);
-    accel_boundary(D, i, xi, pi, a);
-    return a;
-}
-
-// Neighbour sums of the solver iterations may be split over LPP adjacent
-// lanes: lane h of a particle takes neighbours h, h + LPP, ..., and the
-// partial sums are combined by butterfly shuffles in a fixed order (results
-// are deterministic; LPP = 1 is the plain sequential sum). Shorter per-lane
-// chains of dependent gathers keep more loads in flight per wave.
+// Pressure acceleration of particle i (zero unless live), complete in lane
+// hl == 0. The lanes of a particle call this together.
 template <int LPP>
-__device__ __forceinline__ float lane_sum(float v) {
-    if (LPP >= 2) v += __shfl_xor(v, 1, 64);
-    if (LPP >= 4) v += __shfl_xor(v, 2, 64);
-    if (LPP >= 8) v += __shfl_xor(v, 4, 64);
-    return v;
-}
-
-// Calls f(j, ld(j)) for the fluid neighbours of particle i taken by lane
-// hl, the loads ld of four neighbours issued before the first f, so each
-// wave keeps more gathers in flight.
-struct F4x2 {
-    float4 a, b;
-};
-template <int LPP, class LD, class F>
-__device__ __forceinline__ void fluid_pairs(const Dev &D, unsigned i, unsigned hl, unsigned cnt, LD &&ld, F &&f) {
-    fluid_nbrs4<LPP>(
-        D, i, hl, cnt,
-        [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-            const auto a0 = ld(j0);
-            const auto a1 = ld(j1);
-            const auto a2 = ld(j2);
-            const auto a3 = ld(j3);
-            f(j0, a0);
-            f(j1, a1);
-            f(j2, a2);
-            f(j3, a3);
-        },
-        [&](unsigned j) { f(j, ld(j)); });
-}
-
-// Calls f(j) for the fluid neighbours of particle i taken by lane hl.
-template <int LPP, class F>
-__device__ __forceinline__ void fluid_nbrs(const Dev &D, unsigned i, unsigned hl, unsigned cnt, F &&f) {
-    fluid_nbrs4<LPP>(
-        D, i, hl, cnt,
-        [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-            f(j0);
-            f(j1);
-            f(j2);
-            f(j3);
-        },
-        f);
+__device__ __forceinline__ float3 particle_accel(const Dev &D, unsigned i, unsigned hl, bool live,
+                                                 const float *__restrict__ P, float *__restrict__ T) {
+    float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
+    float pi = 0.f, ir = 1.f;
+    float acc[3] = {0.f, 0.f, 0.f};
+    if (live) {
+        xi = D.x[i];
+        pi = P[i];
+        if (D.model) ir = 1.0f / rho0_of(D, i);
+        const F4Gather X(D.x, D.n);
+        fluid_sums<LPP, SumVec>(
+            D, i, hl, D.cf[i], T, acc, loads([&](unsigned j) { return X.all(j); }),
+            [&](unsigned, const auto &q, float *t) { return accel_term(D, xi, pi, q.a, ir, t); });
+    }
+    lanes_join<LPP, SumVec>(acc);
+    if (D.bmode == 1)
+        akinci_sums<LPP, SumAdd<3>>(D, i, hl, live && fabsf(pi) > D.eps ? D.cb[i] : 0u, T, acc,
+                                    [&](const float4 &xb, float *t) {
+                                        float3 r;
+                                        const float g = kernel_G(xi, xb, D.K, r);
+                                        t[0] = pi * (-xb.w * (g * r.x));
+                                        t[1] = pi * (-xb.w * (g * r.y));
+                                        t[2] = pi * (-xb.w * (g * r.z));
+                                        return true;
+                                    });
+    float3 a = make_float3(acc[0], acc[1], acc[2]);
+    if (live && hl == 0) accel_maps(D, i, xi, pi, a);
+    return a;
 }
 
 // The acceleration sweep of block `blk` of a particle range; the single
@@ -397,64 +622,10 @@ __device__ __forceinline__ void accel_sweep(const Dev &D, unsigned blk, int chec
     // computePressureAccel leaves a_p = 0 for particles that are not active
     // (TimeStepDFSPH.cpp:1303-1310)
     const bool live = act && is_active(D, i);
-    const float *__restrict__ P = PRESSURE ? D.p : D.pv;
-    float ax = 0.f, ay = 0.f, az = 0.f, pi = 0.f;
-    float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
-    float ir = 1.f;
-    if (live) {
-        xi = D.x[i];
-        pi = P[i];
-        if (D.model) ir = 1.0f / rho0_of(D, i);
-        const F4Gather X(D.x, D.n);
-        fluid_nbrs4<LPP>(
-            D, i, h, D.cf[i],
-            [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-                const float4 x0 = X.all(j0), x1 = X.all(j1), x2 = X.all(j2), x3 = X.all(j3);
-                accel_pair(D, xi, pi, x0, ax, ay, az, ir);
-                accel_pair(D, xi, pi, x1, ax, ay, az, ir);
-                accel_pair(D, xi, pi, x2, ax, ay, az, ir);
-                accel_pair(D, xi, pi, x3, ax, ay, az, ir);
-            },
-            [&](unsigned j) { accel_pair(D, xi, pi, X.all(j), ax, ay, az, ir); });
-    }
-    if (LPP > 1) {
-        ax = lane_sum<LPP>(ax);
-        ay = lane_sum<LPP>(ay);
-        az = lane_sum<LPP>(az);
-    }
-    if (!act || h != 0) return;
-    if (fabsf(pi) > D.eps) {
-        if (D.bmode == 1) {
-            const unsigned cb = D.cb[i];
-            for (unsigned k = 0; k < cb; k++) {
-                const float4 xb = D.bx[D.nb[(size_t)k * D.stride + i]];
-                float3 r;
-                const float g = kernel_G(xi, xb, D.K, r);
-                ax += pi * (-xb.w * (g * r.x));
-                ay += pi * (-xb.w * (g * r.y));
-                az += pi * (-xb.w * (g * r.z));
-            }
-        } else if (D.bmode == 2) {
-            for (unsigned o = 0; o < D.nvm; o++) {
-                const float4 xb = D.vmb[(size_t)o * D.stride + i];
-                if (!(xb.w > 0.f)) break;
-                float3 r;
-                const float g = kernel_G(xi, xb, D.K, r);
-                ax += pi * (-xb.w * (g * r.x));
-                ay += pi * (-xb.w * (g * r.y));
-                az += pi * (-xb.w * (g * r.z));
-            }
-        } else if (D.bmode == 3) {
-            for (unsigned o = 0; o < D.nvm; o++) {
-                if (!(D.vmb[(size_t)o * D.stride + i].w > 0.f)) break;
-                const float4 gb = D.dmg[(size_t)o * D.stride + i];
-                ax += pi * gb.x;
-                ay += pi * gb.y;
-                az += pi * gb.z;
-            }
-        }
-    }
-    D.ap[i] = make_float4(ax, ay, az, 0.f);
+    __shared__ float plds[PAIR_LDS<LPP, SumVec::NT>];
+    float *const T = pair_part<LPP, SumVec::NT>(plds);
+    const float3 acc = particle_accel<LPP>(D, i, h, live, PRESSURE ? D.p : D.pv, T);
+    if (act && h == 0) D.ap[i] = make_float4(acc.x, acc.y, acc.z, 0.f);
 }
 
 template <bool PRESSURE, int LPP>
@@ -472,13 +643,13 @@ __global__ __launch_bounds__(BLOCK) void kb_accel(const Dev *__restrict__ Ds, co
     accel_sweep<PRESSURE, LPP>(Ds[m.x], m.y, check_done);
 }
 
-// s += (a_i - a_j) . gradW_ij = g_ij ((a_i - a_j) . r_ij)
-__device__ __forceinline__ void aij_acc(float &s, const float4 &xi, const float4 &ai, const float4 &xj,
-                                        const float4 &aj, const KernelConst &K) {
+// t = (g, d) with s += g d: (a_i - a_j) . gradW_ij = g_ij ((a_i - a_j) . r_ij)
+__device__ __forceinline__ bool aij_term(const float4 &xi, const float4 &ai, const float4 &xj, const float4 &aj,
+                                         const KernelConst &K, float *t) {
     float3 r;
-    const float g = kernel_G(xi, xj, K, r);
-    const float d = fmaf(ai.z - aj.z, r.z, fmaf(ai.y - aj.y, r.y, (ai.x - aj.x) * r.x));
-    s = fmaf(g, d, s);
+    t[0] = kernel_G(xi, xj, K, r);
+    t[1] = fmaf(ai.z - aj.z, r.z, fmaf(ai.y - aj.y, r.y, (ai.x - aj.x) * r.x));
+    return true;
 }
 
 // compute_aij_pj (TimeStepDFSPH.cpp:1370-1420) and the Jacobi update of
@@ -487,6 +658,8 @@ __device__ __forceinline__ void aij_acc(float &s, const float4 &xi, const float4
 template <bool PRESSURE, int LPP>
 __device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigned part, int check_done) {
     __shared__ double lds[BLOCK / 64];
+    __shared__ float plds[PAIR_LDS<LPP, SumDot::NT>];
+    float *const T = pair_part<LPP, SumDot::NT>(plds);
     Ctl *C = D.ctl;
     if (check_done && (PRESSURE ? C->done : C->done_v)) return;
     const unsigned t = blk * blockDim.x + threadIdx.x;
@@ -496,40 +669,31 @@ __device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigne
     const bool act = i < D.n && (!PRESSURE || is_active(D, i)) && in_solve(D, i);
     const double h = C->h;
     double err = 0.0, over = 0.0;
-    float s = 0.f;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), ai = xi;
-    unsigned cnt = 0;
+    unsigned cnt = 0, cb = 0;
+    float s = 0.f;
     if (act) {
         xi = D.x[i];
         ai = D.ap[i];
         cnt = D.cf[i];
         const F4Gather X(D.x, D.n), A(D.ap, D.n);
-        fluid_nbrs4<LPP>(
-            D, i, hl, cnt,
-            [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-                const float4 x0 = X.xyz(j0), x1 = X.xyz(j1), x2 = X.xyz(j2), x3 = X.xyz(j3);
-                const float4 a0 = A.xyz(j0), a1 = A.xyz(j1), a2 = A.xyz(j2), a3 = A.xyz(j3);
-                aij_acc(s, xi, ai, x0, a0, D.K);
-                aij_acc(s, xi, ai, x1, a1, D.K);
-                aij_acc(s, xi, ai, x2, a2, D.K);
-                aij_acc(s, xi, ai, x3, a3, D.K);
-            },
-            [&](unsigned j) { aij_acc(s, xi, ai, X.xyz(j), A.xyz(j), D.K); });
+        fluid_sums<LPP, SumDot>(
+            D, i, hl, cnt, T, &s, loads([&](unsigned j) { return X.xyz(j); }, [&](unsigned j) { return A.xyz(j); }),
+            [&](unsigned, const auto &q, float *u) { return aij_term(xi, ai, q.a, q.b, D.K, u); });
     }
-    if (LPP > 1) s = lane_sum<LPP>(s);
+    lanes_join<LPP, SumDot>(&s);
+    s *= D.V;
+    if (act && D.bmode == 1) cb = D.cb[i];
+    if (D.bmode == 1)
+        akinci_sums<LPP, SumAdd<1>>(D, i, hl, cb, T, &s, [&](const float4 &xb, float *u) {
+            float3 r;
+            const float g = kernel_G(xi, xb, D.K, r);
+            u[0] = xb.w * ((ai.x * (g * r.x) + ai.y * (g * r.y)) + ai.z * (g * r.z));
+            return true;
+        });
     if (act && hl == 0) {
-        s *= D.V;
-        unsigned nnb = cnt;
-        if (D.bmode == 1) {
-            const unsigned cb = D.cb[i];
-            nnb += cb;
-            for (unsigned k = 0; k < cb; k++) {
-                const float4 xb = D.bx[D.nb[(size_t)k * D.stride + i]];
-                float3 r;
-                const float g = kernel_G(xi, xb, D.K, r);
-                s += xb.w * (((ai.x * (g * r.x) + ai.y * (g * r.y)) + ai.z * (g * r.z)));
-            }
-        } else if (D.bmode == 2) {
+        const unsigned nnb = cnt + cb;
+        if (D.bmode == 2) {
             for (unsigned o = 0; o < D.nvm; o++) {
                 const float4 xb = D.vmb[(size_t)o * D.stride + i];
                 if (!(xb.w > 0.f)) break;
@@ -577,7 +741,7 @@ __device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigne
 }
 
 template <bool PRESSURE, int LPP>
-__global__ __launch_bounds__(BLOCK) void k_jacobi(Dev D, int check_done) {
+__global__ __launch_bounds__(BLOCK, LPP == 2 ? 7 : 1) void k_jacobi(Dev D, int check_done) {
     jacobi_sweep<PRESSURE, LPP>(D, xcd_block(), blockIdx.x, check_done);
 }
 
@@ -743,29 +907,9 @@ __global__ __launch_bounds__(BLOCK) void k_finish(Dev D) {
     const unsigned i = t / LPP, hl = t % LPP;
     const bool act = i < D.n;
     const bool live = act && is_active(D, i);  // a_p = 0 otherwise (TimeStepDFSPH.cpp:1309)
-    const float *__restrict__ P = PRESSURE ? D.p : D.pv;
-    float3 a = make_float3(0.f, 0.f, 0.f);
-    float pi = 0.f;
-    float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live) {
-        xi = D.x[i];
-        pi = P[i];
-        if (LPP == 1) {
-            a = accel_i(D, i, P);
-        } else {
-            const float ir = D.model ? 1.0f / rho0_of(D, i) : 1.f;
-            const F4Gather X(D.x, D.n);
-            fluid_pairs<LPP>(
-                D, i, hl, D.cf[i], [&](unsigned j) { return X.all(j); },
-                [&](unsigned, const float4 &xj) { accel_pair(D, xi, pi, xj, a.x, a.y, a.z, ir); });
-        }
-    }
-    if (LPP > 1) {
-        a.x = lane_sum<LPP>(a.x);
-        a.y = lane_sum<LPP>(a.y);
-        a.z = lane_sum<LPP>(a.z);
-        if (live && hl == 0) accel_boundary(D, i, xi, pi, a);
-    }
+    __shared__ float plds[PAIR_LDS<LPP, SumVec::NT>];
+    float *const T = pair_part<LPP, SumVec::NT>(plds);
+    const float3 a = particle_accel<LPP>(D, i, hl, live, PRESSURE ? D.p : D.pv, T);
     if (!act || hl != 0) return;
     const float h = (float)D.ctl->h;
     D.ap[i] = make_float4(a.x, a.y, a.z, 0.f);
@@ -997,6 +1141,8 @@ __global__ __launch_bounds__(RBLOCK) void k_body_reduce(Dev D, unsigned nparts) 
 template <bool CLEAR, bool APPLY, bool XSPH, bool CFL, bool VUPD, bool SCALEPV, int LPP>
 __global__ __launch_bounds__(BLOCK) void k_post(Dev D) {
     __shared__ double lds[BLOCK / 64];
+    __shared__ float plds[XSPH ? PAIR_LDS<LPP, SumVecAdd::NT> : 1];
+    float *const T = pair_part<LPP, SumVecAdd::NT>(plds);
     Ctl *C = D.ctl;
     const unsigned t = gtid();
     const unsigned i = t / LPP, hl = t % LPP;
@@ -1008,6 +1154,7 @@ __global__ __launch_bounds__(BLOCK) void k_post(Dev D) {
     float4 vi = make_float4(0.f, 0.f, 0.f, 0.f), xi = vi;
     float sx = 0.f, sy = 0.f, sz = 0.f;  // XSPH fluid sum
     float ux = 0.f, uy = 0.f, uz = 0.f;  // standard viscosity fluid sum
+    float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (act) {
         vi = D.v[i];
         if (XSPH) {
@@ -1016,42 +1163,58 @@ __global__ __launch_bounds__(BLOCK) void k_post(Dev D) {
             const bool xs = cxs != 0.f, sv = csv != 0.f;
             const unsigned mi = D.model ? D.model[i] : 0u;
             const F4Gather X(D.x, D.n), V(D.v, D.n);
-            if (xs || sv)
-                fluid_pairs<LPP>(
-                    D, i, hl, D.cf[i], [&](unsigned j) { return F4x2{X.all(j), V.xyz(j)}; },
-                    [&](unsigned j, const F4x2 &q) {
-                    const float4 &xj = q.a, &vj = q.b;  // xj.w: m_j / rho_j
-                    // each model's viscosity acts within the model
-                    // (forall_fluid_neighbors_in_same_phase, Viscosity_Standard.cpp:271)
-                    if (sv && (!D.model || D.model[j] == mi)) {
-                        // Viscosity_Standard (Viscosity_Standard.cpp:281-289):
-                        // d nu m_j/rho_j (v_ij . x_ij) / (|x_ij|^2 + 0.01 h^2) gradW
-                        float3 r;
-                        const float g = kernel_G(xi, xj, D.K, r);
-                        const float dot = fmaf(vi.z - vj.z, r.z, fmaf(vi.y - vj.y, r.y, (vi.x - vj.x) * r.x));
-                        const float s = csv * xj.w * dot * g *
-                                        __builtin_amdgcn_rcpf(fmaf(0.01f, D.hs2, sqn_fma(r.x, r.y, r.z)));
-                        ux = fmaf(s, r.x, ux);
-                        uy = fmaf(s, r.y, uy);
-                        uz = fmaf(s, r.z, uz);
-                    }
-                    if (xs) {
-                        const float w = kernel_W(xi, xj, D.K);
-                        const float s = invH * cxs * xj.w;
-                        sx -= s * (vi.x - vj.x) * w;
-                        sy -= s * (vi.y - vj.y) * w;
-                        sz -= s * (vi.z - vj.z) * w;
-                    }
+            // Viscosity_Standard (Viscosity_Standard.cpp:281-289), within the
+            // model (forall_fluid_neighbors_in_same_phase, :271):
+            // d nu m_j/rho_j (v_ij . x_ij) / (|x_ij|^2 + 0.01 h^2) gradW
+            auto visc = [&](unsigned j, const auto &q, float *u) {
+                if (!(sv && (!D.model || D.model[j] == mi))) return false;
+                const float4 &xj = q.a, &vj = q.b;  // xj.w: m_j / rho_j
+                float3 r;
+                const float g = kernel_G(xi, xj, D.K, r);
+                const float dot = fmaf(vi.z - vj.z, r.z, fmaf(vi.y - vj.y, r.y, (vi.x - vj.x) * r.x));
+                u[0] = csv * xj.w * dot * g * __builtin_amdgcn_rcpf(fmaf(0.01f, D.hs2, sqn_fma(r.x, r.y, r.z)));
+                u[1] = r.x;
+                u[2] = r.y;
+                u[3] = r.z;
+                return true;
+            };
+            auto xsph = [&](const auto &q, float *u) {
+                if (!xs) return false;
+                const float4 &xj = q.a, &vj = q.b;
+                const float w = kernel_W(xi, xj, D.K);
+                const float s = invH * cxs * xj.w;
+                u[0] = -(s * (vi.x - vj.x) * w);
+                u[1] = -(s * (vi.y - vj.y) * w);
+                u[2] = -(s * (vi.z - vj.z) * w);
+                return true;
+            };
+            const auto ld = loads([&](unsigned j) { return X.all(j); }, [&](unsigned j) { return V.xyz(j); });
+            const unsigned cnt = (xs || sv) ? D.cf[i] : 0u;
+            if constexpr (LPP != ORDERED_LANES)
+                fluid_pairs<LPP>(D, i, hl, cnt, ld, [&](unsigned j, const auto &q) {
+                    float u[4];
+                    if (visc(j, q, u)) sum_terms<SumVec>(u, acc + 3);
+                    if (xsph(q, u)) sum_terms<SumAdd<3>>(u, acc);
+                });
+            else
+                fluid_sums<LPP, SumVecAdd>(D, i, hl, cnt, T, acc, ld, [&](unsigned j, const auto &q, float *u) {
+#pragma unroll
+                    for (int c = 0; c < 7; c++) u[c] = 0.f;
+                    u[7] = 1.f;
+                    visc(j, q, u + 3);
+                    xsph(q, u);
+                    return true;
                 });
         }
     }
-    if (XSPH && LPP > 1) {
-        sx = lane_sum<LPP>(sx);
-        sy = lane_sum<LPP>(sy);
-        sz = lane_sum<LPP>(sz);
-        ux = lane_sum<LPP>(ux);
-        uy = lane_sum<LPP>(uy);
-        uz = lane_sum<LPP>(uz);
+    if (XSPH) {
+        lanes_join<LPP, SumVecAdd>(acc);
+        sx = acc[0];
+        sy = acc[1];
+        sz = acc[2];
+        ux = acc[3];
+        uy = acc[4];
+        uz = acc[5];
     }
     if (act && hl == 0) {
         float4 ai = CLEAR ? make_float4(D.grav.x, D.grav.y, D.grav.z, 0.f) : D.a[i];
@@ -1174,34 +1337,30 @@ __global__ __launch_bounds__(BLOCK) void k_psetup(Dev D) {
     const unsigned t = gtid();
     const unsigned i = t / LPP, hl = t % LPP;
     const bool act = i < D.n;
+    __shared__ float plds[PAIR_LDS<LPP, SumDot::NT>];
+    float *const T = pair_part<LPP, SumDot::NT>(plds);
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), vi = xi;
     float delta = 0.f;
     if (act) {
         xi = D.x[i];
         vi = D.v[i];
         const F4Gather X(D.x, D.n), V(D.v, D.n);
-        fluid_pairs<LPP>(
-            D, i, hl, D.cf[i], [&](unsigned j) { return F4x2{X.xyz(j), V.xyz(j)}; },
-            [&](unsigned, const F4x2 &q) {
-                const float4 &vj = q.b;
-                float3 r;
-                const float g = kernel_G(xi, q.a, D.K, r);
-                delta = fmaf(g, fmaf(vi.z - vj.z, r.z, fmaf(vi.y - vj.y, r.y, (vi.x - vj.x) * r.x)), delta);
-            });
+        fluid_sums<LPP, SumDot>(
+            D, i, hl, D.cf[i], T, &delta, loads([&](unsigned j) { return X.xyz(j); }, [&](unsigned j) { return V.xyz(j); }),
+            [&](unsigned, const auto &q, float *u) { return aij_term(xi, vi, q.a, q.b, D.K, u); });
     }
-    if (LPP > 1) delta = lane_sum<LPP>(delta);
-    if (!act || hl != 0) return;
-    const double h = D.ctl->h;
+    lanes_join<LPP, SumDot>(&delta);
     delta *= D.V;
-    if (D.bmode == 1) {
-        const unsigned cb = D.cb[i];
-        for (unsigned k = 0; k < cb; k++) {
-            const float4 xb = D.bx[D.nb[(size_t)k * D.stride + i]];
+    if (D.bmode == 1)
+        akinci_sums<LPP, SumAdd<1>>(D, i, hl, act ? D.cb[i] : 0u, T, &delta, [&](const float4 &xb, float *u) {
             float3 r;
             const float g = kernel_G(xi, xb, D.K, r);
-            delta += xb.w * ((vi.x * (g * r.x) + vi.y * (g * r.y)) + vi.z * (g * r.z));
-        }
-    } else if (D.bmode == 2) {
+            u[0] = xb.w * ((vi.x * (g * r.x) + vi.y * (g * r.y)) + vi.z * (g * r.z));
+            return true;
+        });
+    if (!act || hl != 0) return;
+    const double h = D.ctl->h;
+    if (D.bmode == 2) {
         for (unsigned o = 0; o < D.nvm; o++) {
             const float4 xb = D.vmb[(size_t)o * D.stride + i];
             if (!(xb.w > 0.f)) break;
@@ -1323,38 +1482,39 @@ __device__ __forceinline__ void weiler_boundary(const Dev &D, unsigned i, const 
     }
 }
 
-// One pair of the operator: with c the pair's coefficient (fluid:
-// d mu m_j / rho_j), adds c g_ij (r r^T) / (|r|^2 + 0.01 h^2) to the block
-// diagonal m (xx xy xz yy yz zz; DIAG) and c (dv . r) / (|r|^2 + 0.01 h^2)
-// g_ij r to the product a (AV).
+// Terms of one pair of the operator: with c the pair's coefficient (fluid:
+// d mu m_j / rho_j), weiler_av gives t = (s, r) with s r = c (dv . r) /
+// (|r|^2 + 0.01 h^2) g_ij r, its part of the product, and weiler_diag
+// t = (u, r) with u r^T = c g_ij (r r^T) / (|r|^2 + 0.01 h^2), its part of
+// the block diagonal (xx xy xz yy yz zz).
 // The quotients use the hardware reciprocal (1 ulp) in place of a
 // correctly rounded division: a per-pair term carries rounding at the
 // 1e-7 level either way.
-template <bool DIAG, bool AV>
-__device__ __forceinline__ void weiler_pair(const Dev &D, const float4 &xi, const float4 &xj, float c, const float4 &vi,
-                                            const float4 &vj, float *m, float &ax, float &ay, float &az) {
+__device__ __forceinline__ bool weiler_av(const Dev &D, const float4 &xi, const float4 &xj, float c, const float4 &vi,
+                                          const float4 &vj, float *t) {
     float3 r;
     const float g = kernel_G(xi, xj, D.K, r);
     const float iden = __builtin_amdgcn_rcpf(fmaf(0.01f, D.hs2, sqn_fma(r.x, r.y, r.z)));
-    if (DIAG) {
-        const float s = c * iden * g;  // c g / den
-        const float sx = s * r.x, sy = s * r.y, sz = s * r.z;
-        m[0] = fmaf(sx, r.x, m[0]);
-        m[1] = fmaf(sx, r.y, m[1]);
-        m[2] = fmaf(sx, r.z, m[2]);
-        m[3] = fmaf(sy, r.y, m[3]);
-        m[4] = fmaf(sy, r.z, m[4]);
-        m[5] = fmaf(sz, r.z, m[5]);
-    }
-    if (AV) {
-        const float dot = fmaf(vi.z - vj.z, r.z, fmaf(vi.y - vj.y, r.y, (vi.x - vj.x) * r.x));
-        const float s = c * dot * iden * g;
-        ax = fmaf(s, r.x, ax);
-        ay = fmaf(s, r.y, ay);
-        az = fmaf(s, r.z, az);
-    }
+    const float dot = fmaf(vi.z - vj.z, r.z, fmaf(vi.y - vj.y, r.y, (vi.x - vj.x) * r.x));
+    t[0] = c * dot * iden * g;
+    t[1] = r.x;
+    t[2] = r.y;
+    t[3] = r.z;
+    return true;
 }
-
+__device__ __forceinline__ bool weiler_diag(const Dev &D, const float4 &xi, const float4 &xj, float c, float *t) {
+    float3 r;
+    const float g = kernel_G(xi, xj, D.K, r);
+    const float iden = __builtin_amdgcn_rcpf(fmaf(0.01f, D.hs2, sqn_fma(r.x, r.y, r.z)));
+    const float s = c * iden * g;  // c g / den
+    t[0] = s * r.x;
+    t[1] = s * r.y;
+    t[2] = s * r.z;
+    t[3] = r.x;
+    t[4] = r.y;
+    t[5] = r.z;
+    return true;
+}
 __device__ __forceinline__ float3 minv_apply(const Dev &D, unsigned i, const float3 &r) {
     const float4 a = D.minv[2 * i], b = D.minv[2 * i + 1];
     return make_float3((a.x * r.x + a.y * r.y) + a.z * r.z, (a.y * r.x + a.w * r.y) + b.x * r.z,
@@ -1367,33 +1527,29 @@ __device__ __forceinline__ float3 minv_apply(const Dev &D, unsigned i, const flo
 // positions' w holds m_j / rho_j.
 template <int LPP>
 __device__ __forceinline__ float3 weiler_Av(const Dev &D, unsigned i, unsigned hl, bool act,
-                                            const float4 *__restrict__ vec) {
+                                            const float4 *__restrict__ vec, float *__restrict__ T) {
     const float dd = 10.0f;
-    float ax = 0.f, ay = 0.f, az = 0.f;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), vi = xi;
+    float a[3] = {0.f, 0.f, 0.f};
     if (act) {
         xi = D.x[i];
         vi = vec[i];
         const F4Gather X(D.x, D.n), Vc(vec, D.n);
-        fluid_pairs<LPP>(
-            D, i, hl, D.cf[i], [&](unsigned j) { return F4x2{X.all(j), Vc.xyz(j)}; },
-            [&](unsigned, const F4x2 &q) {
-                weiler_pair<false, true>(D, xi, q.a, dd * D.mu * q.a.w, vi, q.b, nullptr, ax, ay, az);
-            });
+        fluid_sums<LPP, SumVec>(
+            D, i, hl, D.cf[i], T, a, loads([&](unsigned j) { return X.all(j); }, [&](unsigned j) { return Vc.xyz(j); }),
+            [&](unsigned, const auto &q, float *t) { return weiler_av(D, xi, q.a, dd * D.mu * q.a.w, vi, q.b, t); });
     }
-    if (LPP > 1) {
-        ax = lane_sum<LPP>(ax);
-        ay = lane_sum<LPP>(ay);
-        az = lane_sum<LPP>(az);
-    }
+    lanes_join<LPP, SumVec>(a);
     if (!act || hl != 0) return make_float3(0.f, 0.f, 0.f);
     const float rhoi = D.rho[i];
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
     weiler_boundary(D, i, xi, rhoi, [&](const float4 &xs, float c) {
-        weiler_pair<false, true>(D, xi, xs, c, vi, z4, nullptr, ax, ay, az);
+        float t[4];
+        weiler_av(D, xi, xs, c, vi, z4, t);
+        sum_terms<SumVec>(t, a);
     });
     const float f = (float)D.ctl->h / rhoi;
-    return make_float3(vi.x - f * ax, vi.y - f * ay, vi.z - f * az);
+    return make_float3(vi.x - f * a[0], vi.y - f * a[1], vi.z - f * a[2]);
 }
 
 // Set-up of the Weiler2018 solve, in Eigen's order (ConjugateGradient.h:43-70):
@@ -1418,35 +1574,33 @@ __global__ __launch_bounds__(BLOCK) void k_weiler_r0(Dev D) {
     const unsigned t = gtid();
     const unsigned i = t / LPP, hl = t % LPP;
     const bool act = i < D.n;
+    __shared__ float plds[PAIR_LDS<LPP, SumVec::NT>];
+    float *const T = pair_part<LPP, SumVec::NT>(plds);
     const float dd = 10.0f;
-    float ax = 0.f, ay = 0.f, az = 0.f;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), x0i = xi, vi = xi;
+    float a[3] = {0.f, 0.f, 0.f};
     if (act) {
         xi = D.x[i];
         vi = D.v[i];
         const float4 vd = D.vdiff[i];
         x0i = make_float4(vi.x + vd.x, vi.y + vd.y, vi.z + vd.z, 0.f);
         const F4Gather X(D.x, D.n), X0(D.cgx, D.n);
-        fluid_pairs<LPP>(
-            D, i, hl, D.cf[i], [&](unsigned j) { return F4x2{X.all(j), X0.xyz(j)}; },
-            [&](unsigned, const F4x2 &q) {
-                weiler_pair<false, true>(D, xi, q.a, dd * D.mu * q.a.w, x0i, q.b, nullptr, ax, ay, az);
-            });
+        fluid_sums<LPP, SumVec>(
+            D, i, hl, D.cf[i], T, a, loads([&](unsigned j) { return X.all(j); }, [&](unsigned j) { return X0.xyz(j); }),
+            [&](unsigned, const auto &q, float *u) { return weiler_av(D, xi, q.a, dd * D.mu * q.a.w, x0i, q.b, u); });
     }
-    if (LPP > 1) {
-        ax = lane_sum<LPP>(ax);
-        ay = lane_sum<LPP>(ay);
-        az = lane_sum<LPP>(az);
-    }
+    lanes_join<LPP, SumVec>(a);
     double b2 = 0.0, r2 = 0.0;
     if (act && hl == 0) {
         const float rhoi = D.rho[i];
         const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
         weiler_boundary(D, i, xi, rhoi, [&](const float4 &xs, float c) {
-            weiler_pair<false, true>(D, xi, xs, c, x0i, z4, nullptr, ax, ay, az);
+            float u[4];
+            weiler_av(D, xi, xs, c, x0i, z4, u);
+            sum_terms<SumVec>(u, a);
         });
         const float fa = (float)D.ctl->h / rhoi;
-        const float3 Ax = make_float3(x0i.x - fa * ax, x0i.y - fa * ay, x0i.z - fa * az);
+        const float3 Ax = make_float3(x0i.x - fa * a[0], x0i.y - fa * a[1], x0i.z - fa * a[2]);
         const float3 r = make_float3(vi.x - Ax.x, vi.y - Ax.y, vi.z - Ax.z);
         D.cgr[i] = make_float4(r.x, r.y, r.z, 0.f);
         b2 = ((double)vi.x * vi.x + (double)vi.y * vi.y) + (double)vi.z * vi.z;
@@ -1495,28 +1649,25 @@ __global__ __launch_bounds__(BLOCK) void k_weiler_precond(Dev D) {
     const unsigned i = t / LPP, hl = t % LPP;
     const bool act = i < D.n;
     const float dd = 10.0f;
+    __shared__ float plds[PAIR_LDS<LPP, SumSym::NT>];
+    float *const T = pair_part<LPP, SumSym::NT>(plds);
     float m[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float ax = 0.f, ay = 0.f, az = 0.f;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 z4 = xi;
     if (act) {
         xi = D.x[i];
         const F4Gather X(D.x, D.n);
-        fluid_pairs<LPP>(
-            D, i, hl, D.cf[i], [&](unsigned j) { return X.all(j); },
-            [&](unsigned, const float4 &xj) {
-                weiler_pair<true, false>(D, xi, xj, dd * D.mu * xj.w, z4, z4, m, ax, ay, az);
-            });
+        fluid_sums<LPP, SumSym>(
+            D, i, hl, D.cf[i], T, m, loads([&](unsigned j) { return X.all(j); }),
+            [&](unsigned, const auto &q, float *u) { return weiler_diag(D, xi, q.a, dd * D.mu * q.a.w, u); });
     }
-    if (LPP > 1) {
-#pragma unroll
-        for (int q = 0; q < 6; q++) m[q] = lane_sum<LPP>(m[q]);
-    }
+    lanes_join<LPP, SumSym>(m);
     double rz = 0.0;
     if (act && hl == 0) {
         const float rhoi = D.rho[i];
         weiler_boundary(D, i, xi, rhoi, [&](const float4 &xs, float c) {
-            weiler_pair<true, false>(D, xi, xs, c, z4, z4, m, ax, ay, az);
+            float u[6];
+            weiler_diag(D, xi, xs, c, u);
+            sum_terms<SumSym>(u, m);
         });
         const double f = (double)D.ctl->h / (double)rhoi;
         double md[6] = {1.0 - f * m[0], -f * m[1], -f * m[2], 1.0 - f * m[3], -f * m[4], 1.0 - f * m[5]};
@@ -1556,8 +1707,10 @@ __global__ __launch_bounds__(BLOCK) void k_cg_matvec(Dev D) {
     const unsigned tid = gtid();
     const unsigned i = tid / LPP, hl = tid % LPP;
     const bool act = i < D.n;
+    __shared__ float plds[PAIR_LDS<LPP, SumVec::NT>];
+    float *const T = pair_part<LPP, SumVec::NT>(plds);
     double pt = 0.0;
-    const float3 t = weiler_Av<LPP>(D, i, hl, act, D.cgp);
+    const float3 t = weiler_Av<LPP>(D, i, hl, act, D.cgp, T);
     if (act && hl == 0) {
         D.cgt[i] = make_float4(t.x, t.y, t.z, 0.f);
         const float4 p = D.cgp[i];
@@ -1689,9 +1842,10 @@ __global__ __launch_bounds__(RBLOCK) void k_kref_reduce(Dev D, unsigned nparts) 
 // weighted neighbourhood mean, the previous-step stiffness and its mean (both
 // relative to the step's largest), the boundary volume (relative to V) and
 // the neighbour count / 40.
-template <bool PRESSURE>
+template <bool PRESSURE, int LPP>
 __global__ __launch_bounds__(BLOCK) void k_features(Dev D) {
-    const unsigned i = gtid();
+    const unsigned t = gtid();
+    const unsigned i = t / LPP, hl = t % LPP;
     if (i >= D.n) return;
     const double h = D.ctl->h;
     const float sh = PRESSURE ? 1.0f : (float)h;
@@ -1700,35 +1854,33 @@ __global__ __launch_bounds__(BLOCK) void k_features(Dev D) {
     const float ik = kref > 0.f ? 1.0f / kref : 0.0f;
     const float4 xi = D.x[i];
     const float src_i = (D.radv[i] - off) * sh;
+    __shared__ float plds[PAIR_LDS<LPP, 3>];
+    float *const T = pair_part<LPP, 3>(plds);
     const float w0 = D.V * D.K.W0;
-    float wsum = w0, ssrc = w0 * src_i, sk = w0 * D.kprev[i];
-    const unsigned cnt = D.cf[i];
-    auto add = [&](const float4 &xj, float rj, float kj) {
-        const float w = D.V * kernel_W(xi, xj, D.K);
-        wsum += w;
-        ssrc += w * ((rj - off) * sh);
-        sk += w * kj;
-    };
+    float acc[3] = {w0, w0 * src_i, w0 * D.kprev[i]};
+    const unsigned cnt = D.cf[i], cb = D.bmode == 1 ? D.cb[i] : 0u;
     const F4Gather X(D.x, D.n);
-    fluid_nbrs4<1>(
-        D, i, 0, cnt,
-        [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-            const float4 x0 = X.xyz(j0), x1 = X.xyz(j1), x2 = X.xyz(j2), x3 = X.xyz(j3);
-            const float r0 = D.radv[j0], r1 = D.radv[j1], r2 = D.radv[j2], r3 = D.radv[j3];
-            const float k0 = D.kprev[j0], k1 = D.kprev[j1], k2 = D.kprev[j2], k3 = D.kprev[j3];
-            add(x0, r0, k0);
-            add(x1, r1, k1);
-            add(x2, r2, k2);
-            add(x3, r3, k3);
-        },
-        [&](unsigned j) { add(X.xyz(j), D.radv[j], D.kprev[j]); });
+    fluid_sums<LPP, SumAdd<3>>(
+        D, i, hl, cnt, T, acc,
+        loads([&](unsigned j) { return X.xyz(j); }, [&](unsigned j) { return D.radv[j]; },
+              [&](unsigned j) { return D.kprev[j]; }),
+        [&](unsigned, const auto &q, float *u) {
+            const float w = D.V * kernel_W(xi, q.a, D.K);
+            u[0] = w;
+            u[1] = w * ((q.b - off) * sh);
+            u[2] = w * q.c;
+            return true;
+        });
+    const float wsum = acc[0], ssrc = acc[1], sk = acc[2];
     float bvol = 0.f;
-    unsigned nnb = cnt;
-    if (D.bmode == 1) {
-        const unsigned cb = D.cb[i];
-        nnb += cb;
-        for (unsigned k = 0; k < cb; k++) bvol += D.bx[D.nb[(size_t)k * D.stride + i]].w;
-    } else if (D.bmode == 2 || D.bmode == 3) {
+    const unsigned nnb = cnt + cb;
+    if (D.bmode == 1)
+        akinci_sums<LPP, SumAdd<1>>(D, i, hl, cb, T, &bvol, [&](const float4 &xb, float *u) {
+            u[0] = xb.w;
+            return true;
+        });
+    if (hl != 0) return;
+    if (D.bmode == 2 || D.bmode == 3) {
         for (unsigned o = 0; o < D.nvm; o++) {
             const float w = D.vmb[(size_t)o * D.stride + i].w;
             if (!(w > 0.f)) break;
@@ -1777,182 +1929,165 @@ __global__ __launch_bounds__(BLOCK) void k_pred_start(Dev D) {
 }
 
 // Pressure accelerations of both candidate starts (plain P, predicted Q).
-template <bool PRESSURE>
+template <bool PRESSURE, int LPP>
 __global__ __launch_bounds__(BLOCK) void k_accel2(Dev D) {
-    const unsigned i = gtid();
+    const unsigned t = gtid();
+    const unsigned i = t / LPP, hl = t % LPP;
     if (i >= D.n) return;
     if (!is_active(D, i)) {
-        D.ap[i] = D.ap2[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (hl == 0) D.ap[i] = D.ap2[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         return;
     }
     const float *__restrict__ P = PRESSURE ? D.p : D.pv;
     const float *__restrict__ Q = D.pred;
     const float4 xi = D.x[i];
     const float pi = P[i], qi = Q[i];
-    float ax = 0.f, ay = 0.f, az = 0.f, bxx = 0.f, byy = 0.f, bzz = 0.f;
-    const unsigned cnt = D.cf[i];
-    auto pair = [&](const float4 &xj, float pj, float qj) {
-        const float ps = pi + pj, qs = qi + qj;
-        const bool a = fabsf(ps) > D.eps, b = fabsf(qs) > D.eps;
-        if (a || b) {
-            float3 r;
-            const float g = kernel_G(xi, xj, D.K, r);
-            const float gx = -D.V * (g * r.x), gy = -D.V * (g * r.y), gz = -D.V * (g * r.z);
-            if (a) {
-                ax += ps * gx;
-                ay += ps * gy;
-                az += ps * gz;
-            }
-            if (b) {
-                bxx += qs * gx;
-                byy += qs * gy;
-                bzz += qs * gz;
-            }
-        }
-    };
+    __shared__ float plds[PAIR_LDS<LPP, 6>];
+    float *const T = pair_part<LPP, 6>(plds);
     // the fallback start P of a neighbour comes with its position: k_pred_start
     // wrote it into the w component as well
     const F4Gather X(D.x, D.n);
-    fluid_nbrs4<1>(
-        D, i, 0, cnt,
-        [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-            const float4 x0 = X.all(j0), x1 = X.all(j1), x2 = X.all(j2), x3 = X.all(j3);
-            const float q0 = Q[j0], q1 = Q[j1], q2 = Q[j2], q3 = Q[j3];
-            pair(x0, x0.w, q0);
-            pair(x1, x1.w, q1);
-            pair(x2, x2.w, q2);
-            pair(x3, x3.w, q3);
-        },
-        [&](unsigned j) {
-            const float4 xj = X.all(j);
-            pair(xj, xj.w, Q[j]);
+    float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    fluid_sums<LPP, SumAdd<6>>(
+        D, i, hl, D.cf[i], T, acc, loads([&](unsigned j) { return X.all(j); }, [&](unsigned j) { return Q[j]; }),
+        [&](unsigned, const auto &n, float *u) {
+            const float ps = pi + n.a.w, qs = qi + n.b;
+            const bool a = fabsf(ps) > D.eps, b = fabsf(qs) > D.eps;
+            if (!(a || b)) return false;
+            float3 r;
+            const float g = kernel_G(xi, n.a, D.K, r);
+            const float gx = -D.V * (g * r.x), gy = -D.V * (g * r.y), gz = -D.V * (g * r.z);
+            u[0] = a ? ps * gx : 0.f;
+            u[1] = a ? ps * gy : 0.f;
+            u[2] = a ? ps * gz : 0.f;
+            u[3] = b ? qs * gx : 0.f;
+            u[4] = b ? qs * gy : 0.f;
+            u[5] = b ? qs * gz : 0.f;
+            return true;
         });
     const bool bp = fabsf(pi) > D.eps, bq = fabsf(qi) > D.eps;
-    if (bp || bq) {
-        auto bterm = [&](const float4 &xb) {
-            float3 r;
-            const float g = kernel_G(xi, xb, D.K, r);
-            const float gx = -xb.w * (g * r.x), gy = -xb.w * (g * r.y), gz = -xb.w * (g * r.z);
+    auto bterm = [&](const float4 &xb, float *u) {
+        float3 r;
+        const float g = kernel_G(xi, xb, D.K, r);
+        const float gx = -xb.w * (g * r.x), gy = -xb.w * (g * r.y), gz = -xb.w * (g * r.z);
+        u[0] = bp ? pi * gx : 0.f;
+        u[1] = bp ? pi * gy : 0.f;
+        u[2] = bp ? pi * gz : 0.f;
+        u[3] = bq ? qi * gx : 0.f;
+        u[4] = bq ? qi * gy : 0.f;
+        u[5] = bq ? qi * gz : 0.f;
+        return true;
+    };
+    if (D.bmode == 1) {
+        akinci_sums<LPP, SumAdd<6>>(D, i, hl, (bp || bq) ? D.cb[i] : 0u, T, acc, bterm);
+    } else if (D.bmode == 2 && (bp || bq) && hl == 0) {
+        for (unsigned o = 0; o < D.nvm; o++) {
+            const float4 xb = D.vmb[(size_t)o * D.stride + i];
+            if (!(xb.w > 0.f)) break;
+            float u[6];
+            bterm(xb, u);
+            sum_terms<SumAdd<6>>(u, acc);
+        }
+    } else if (D.bmode == 3 && (bp || bq) && hl == 0) {
+        for (unsigned o = 0; o < D.nvm; o++) {
+            if (!(D.vmb[(size_t)o * D.stride + i].w > 0.f)) break;
+            const float4 gb = D.dmg[(size_t)o * D.stride + i];
             if (bp) {
-                ax += pi * gx;
-                ay += pi * gy;
-                az += pi * gz;
+                acc[0] += pi * gb.x;
+                acc[1] += pi * gb.y;
+                acc[2] += pi * gb.z;
             }
             if (bq) {
-                bxx += qi * gx;
-                byy += qi * gy;
-                bzz += qi * gz;
-            }
-        };
-        if (D.bmode == 1) {
-            const unsigned cb = D.cb[i];
-            for (unsigned k = 0; k < cb; k++) bterm(D.bx[D.nb[(size_t)k * D.stride + i]]);
-        } else if (D.bmode == 2) {
-            for (unsigned o = 0; o < D.nvm; o++) {
-                const float4 xb = D.vmb[(size_t)o * D.stride + i];
-                if (!(xb.w > 0.f)) break;
-                bterm(xb);
-            }
-        } else if (D.bmode == 3) {
-            for (unsigned o = 0; o < D.nvm; o++) {
-                if (!(D.vmb[(size_t)o * D.stride + i].w > 0.f)) break;
-                const float4 gb = D.dmg[(size_t)o * D.stride + i];
-                if (bp) {
-                    ax += pi * gb.x;
-                    ay += pi * gb.y;
-                    az += pi * gb.z;
-                }
-                if (bq) {
-                    bxx += qi * gb.x;
-                    byy += qi * gb.y;
-                    bzz += qi * gb.z;
-                }
+                acc[3] += qi * gb.x;
+                acc[4] += qi * gb.y;
+                acc[5] += qi * gb.z;
             }
         }
     }
-    D.ap[i] = make_float4(ax, ay, az, 0.f);
-    D.ap2[i] = make_float4(bxx, byy, bzz, 0.f);
+    if (hl != 0) return;
+    D.ap[i] = make_float4(acc[0], acc[1], acc[2], 0.f);
+    D.ap2[i] = make_float4(acc[3], acc[4], acc[5], 0.f);
 }
 
 // First Jacobi iteration from the per-particle better of the two starts: the
 // one with the smaller initial residual |s - (A p)_i| is kept and updated as
 // in pressureSolveIteration / divergenceSolveIteration.
-template <bool PRESSURE>
+template <bool PRESSURE, int LPP>
 __global__ __launch_bounds__(BLOCK) void k_jacobi2(Dev D) {
     __shared__ double lds[BLOCK / 64];
+    __shared__ float plds[PAIR_LDS<LPP, 2>];
+    float *const T = pair_part<LPP, 2>(plds);
     Ctl *C = D.ctl;
-    const unsigned i = gtid();
+    const unsigned t = gtid();
+    const unsigned i = t / LPP, hl = t % LPP;
     const double h = C->h;
     double err = 0.0, over = 0.0;
     bool took = false;
+    // the lanes of a particle take this branch together
     if (i < D.n && (!PRESSURE || is_active(D, i))) {
         const float4 xi = D.x[i], ai = D.ap[i], bi = D.ap2[i];
-        float s1 = 0.f, s2 = 0.f;
-        const unsigned cnt = D.cf[i];
-        auto pair = [&](const float4 &xj, const float4 &aj, const float4 &bj) {
-            float3 r;
-            const float g = kernel_G(xi, xj, D.K, r);
-            const float gx = g * r.x, gy = g * r.y, gz = g * r.z;
-            s1 += ((ai.x - aj.x) * gx + (ai.y - aj.y) * gy) + (ai.z - aj.z) * gz;
-            s2 += ((bi.x - bj.x) * gx + (bi.y - bj.y) * gy) + (bi.z - bj.z) * gz;
-        };
+        float s[2] = {0.f, 0.f};
+        const unsigned cnt = D.cf[i], cb = D.bmode == 1 ? D.cb[i] : 0u;
         const F4Gather X(D.x, D.n), A(D.ap, D.n), A2(D.ap2, D.n);
-        fluid_nbrs4<1>(
-            D, i, 0, cnt,
-            [&](unsigned j0, unsigned j1, unsigned j2, unsigned j3) {
-                const float4 x0 = X.xyz(j0), x1 = X.xyz(j1), x2 = X.xyz(j2), x3 = X.xyz(j3);
-                const float4 a0 = A.xyz(j0), a1 = A.xyz(j1), a2 = A.xyz(j2), a3 = A.xyz(j3);
-                const float4 b0 = A2.xyz(j0), b1 = A2.xyz(j1), b2 = A2.xyz(j2), b3 = A2.xyz(j3);
-                pair(x0, a0, b0);
-                pair(x1, a1, b1);
-                pair(x2, a2, b2);
-                pair(x3, a3, b3);
-            },
-            [&](unsigned j) { pair(X.xyz(j), A.xyz(j), A2.xyz(j)); });
-        s1 *= D.V;
-        s2 *= D.V;
-        unsigned nnb = cnt;
-        auto bterm = [&](const float4 &xb) {
+        fluid_sums<LPP, SumAdd<2>>(
+            D, i, hl, cnt, T, s,
+            loads([&](unsigned j) { return X.xyz(j); }, [&](unsigned j) { return A.xyz(j); },
+                  [&](unsigned j) { return A2.xyz(j); }),
+            [&](unsigned, const auto &q, float *u) {
+                float3 r;
+                const float g = kernel_G(xi, q.a, D.K, r);
+                const float gx = g * r.x, gy = g * r.y, gz = g * r.z;
+                u[0] = ((ai.x - q.b.x) * gx + (ai.y - q.b.y) * gy) + (ai.z - q.b.z) * gz;
+                u[1] = ((bi.x - q.c.x) * gx + (bi.y - q.c.y) * gy) + (bi.z - q.c.z) * gz;
+                return true;
+            });
+        s[0] *= D.V;
+        s[1] *= D.V;
+        const unsigned nnb = cnt + cb;
+        auto bterm = [&](const float4 &xb, float *u) {
             float3 r;
             const float g = kernel_G(xi, xb, D.K, r);
             const float gx = g * r.x, gy = g * r.y, gz = g * r.z;
-            s1 += xb.w * ((ai.x * gx + ai.y * gy) + ai.z * gz);
-            s2 += xb.w * ((bi.x * gx + bi.y * gy) + bi.z * gz);
+            u[0] = xb.w * ((ai.x * gx + ai.y * gy) + ai.z * gz);
+            u[1] = xb.w * ((bi.x * gx + bi.y * gy) + bi.z * gz);
+            return true;
         };
         if (D.bmode == 1) {
-            const unsigned cb = D.cb[i];
-            nnb += cb;
-            for (unsigned k = 0; k < cb; k++) bterm(D.bx[D.nb[(size_t)k * D.stride + i]]);
-        } else if (D.bmode == 2) {
+            akinci_sums<LPP, SumAdd<2>>(D, i, hl, cb, T, s, bterm);
+        } else if (D.bmode == 2 && hl == 0) {
             for (unsigned o = 0; o < D.nvm; o++) {
                 const float4 xb = D.vmb[(size_t)o * D.stride + i];
                 if (!(xb.w > 0.f)) break;
-                bterm(xb);
+                float u[2];
+                bterm(xb, u);
+                sum_terms<SumAdd<2>>(u, s);
             }
-        } else if (D.bmode == 3) {
+        } else if (D.bmode == 3 && hl == 0) {
             for (unsigned o = 0; o < D.nvm; o++) {
                 if (!(D.vmb[(size_t)o * D.stride + i].w > 0.f)) break;
                 const float4 gb = D.dmg[(size_t)o * D.stride + i];
-                s1 -= (ai.x * gb.x + ai.y * gb.y) + ai.z * gb.z;
-                s2 -= (bi.x * gb.x + bi.y * gb.y) + bi.z * gb.z;
+                s[0] -= (ai.x * gb.x + ai.y * gb.y) + ai.z * gb.z;
+                s[1] -= (bi.x * gb.x + bi.y * gb.y) + bi.z * gb.z;
             }
         }
-        const float sc = PRESSURE ? (float)(h * h) : (float)h;
-        const float si = PRESSURE ? 1.0f - D.radv[i] : -D.radv[i];
-        const float r1 = si - s1 * sc, r2 = si - s2 * sc;
-        took = fabsf(r2) < fabsf(r1);
-        const float start = took ? D.pred[i] : (PRESSURE ? D.p[i] : D.pv[i]);
-        const float rr = took ? r2 : r1;
-        float res = fminf(rr, 0.0f);
-        if (!PRESSURE && nnb < 20u) res = 0.0f;
-        const float pn = fmaxf(start - 0.5f * rr * D.alpha[i], 0.0f);
-        if (PRESSURE)
-            D.p[i] = pn;
-        else
-            D.pv[i] = pn;
-        reinterpret_cast<float *>(D.x + i)[3] = pn;
-        err = -(double)D.rho0 * (double)res;
-        if (pn > 0.0f && rr > 0.0f && (PRESSURE || nnb >= 20u)) over = (double)D.rho0 * (double)rr;
+        if (hl == 0) {
+            const float sc = PRESSURE ? (float)(h * h) : (float)h;
+            const float si = PRESSURE ? 1.0f - D.radv[i] : -D.radv[i];
+            const float r1 = si - s[0] * sc, r2 = si - s[1] * sc;
+            took = fabsf(r2) < fabsf(r1);
+            const float start = took ? D.pred[i] : (PRESSURE ? D.p[i] : D.pv[i]);
+            const float rr = took ? r2 : r1;
+            float res = fminf(rr, 0.0f);
+            if (!PRESSURE && nnb < 20u) res = 0.0f;
+            const float pn = fmaxf(start - 0.5f * rr * D.alpha[i], 0.0f);
+            if (PRESSURE)
+                D.p[i] = pn;
+            else
+                D.pv[i] = pn;
+            reinterpret_cast<float *>(D.x + i)[3] = pn;
+            err = -(double)D.rho0 * (double)res;
+            if (pn > 0.0f && rr > 0.0f && (PRESSURE || nnb >= 20u)) over = (double)D.rho0 * (double)rr;
+        }
     }
     const double bs = block_sum(err, lds);
     const double bo = block_sum(over, lds);
@@ -2245,7 +2380,9 @@ void DFSPH::alloc_particles() {
     }
     cf_.reserve(S);
     cb_.reserve(S);
-    partial_.reserve(12 * (size_t)nblocks(S) + 64);  // up to three values per block of up to 4 lanes per particle
+    // up to three values per block of the sweeps, which have up to 4 lanes
+    // per particle, 16 for small counts (small_lanes)
+    partial_.reserve(std::max(12 * (size_t)nblocks(S), 48 * (size_t)nblocks(SMALL_PARTICLES)) + 64);
     if (initialized_ && (mode_[0] || mode_[1] || stride_s_[0] || stride_s_[1])) ensure_learn_buffers();
     if (P.viscosity_method == SPH_VISCOSITY_WEILER2018) {
         minv_.reserve(2 * S);
@@ -2448,8 +2585,20 @@ void DFSPH::build_lists() {
     have_lists_ = true;
 }
 
+// Lanes per particle of a count too small to time. The two give the same
+// sums bit for bit, so the rule only weighs time: shared pairs hide the
+// memory latency of a nearly idle GPU and cost three times the instructions.
+// Whole steps (us), one lane / shared, Akinci walls and plain start: 2,197
+// particles 550 / 407, 12,167 particles 895 / 687, 32,768 particles 1307 /
+// 1203, 50,653 particles 1335 / 1425. Eight scenes of 20k-80k particles
+// stepped together (24.4 / 28.0 ms for six steps) fill the GPU with one lane
+// each, so a scene counts with those it is stepped with.
+constexpr size_t ORDERED_MAX = 40960;
+static int small_lanes(size_t n) { return n <= ORDERED_MAX ? ORDERED_LANES : 1; }
+
 void DFSPH::neighborhood_search() {
     if (!initialized_) init();
+    if (!lpp_fixed_ && !timed_) lpp_ = lppA_ = small_lanes(std::max(n_, company_));
     k_set_hstep<<<1, 1, 0, stream>>>(ctl_.get());
     const unsigned n = (unsigned)n_;
     fsort_.sort(stream, x_.get(), n, grid_, timer);
@@ -2552,10 +2701,23 @@ void DFSPH::volume_maps(const float4 *xin, const unsigned *skip, const int *stop
         TimedScope ts_(timer, stream, name);                                       \
         const int l_ = (lanes);                                                    \
         const unsigned nb_ = nblocks((size_t)n_ * l_);                             \
-        if (l_ == 4)                                                               \
+        if (l_ == ORDERED_LANES)                                                   \
+            K<__VA_ARGS__, ORDERED_LANES><<<nb_, BLOCK, 0, stream>>>(D);           \
+        else if (l_ == 4)                                                          \
             K<__VA_ARGS__, 4><<<nb_, BLOCK, 0, stream>>>(D);                       \
         else if (l_ == 2)                                                          \
             K<__VA_ARGS__, 2><<<nb_, BLOCK, 0, stream>>>(D);                       \
+        else                                                                       \
+            K<__VA_ARGS__, 1><<<nb_, BLOCK, 0, stream>>>(D);                       \
+        SPH_HIP(hipGetLastError());                                                \
+    } while (0)
+// The same for the sweeps that keep the plain sequential sum at every count.
+#define LAUNCH_SEQ(name, K, ...)                                                   \
+    do {                                                                           \
+        TimedScope ts_(timer, stream, name);                                       \
+        const unsigned nb_ = nblocks((size_t)n_ * seq_lanes());                    \
+        if (seq_lanes() == ORDERED_LANES)                                          \
+            K<__VA_ARGS__, ORDERED_LANES><<<nb_, BLOCK, 0, stream>>>(D);           \
         else                                                                       \
             K<__VA_ARGS__, 1><<<nb_, BLOCK, 0, stream>>>(D);                       \
         SPH_HIP(hipGetLastError());                                                \
@@ -2568,7 +2730,9 @@ void DFSPH::volume_maps(const float4 *xin, const unsigned *skip, const int *stop
     do {                                                                           \
         TimedScope ts_(timer, stream, name);                                       \
         const unsigned nb_ = nblocks((size_t)n_ * lpp_);                           \
-        if (lpp_ == 4)                                                             \
+        if (lpp_ == ORDERED_LANES)                                                 \
+            K<ORDERED_LANES><<<nb_, BLOCK, 0, stream>>>(D);                        \
+        else if (lpp_ == 4)                                                        \
             K<4><<<nb_, BLOCK, 0, stream>>>(D);                                    \
         else if (lpp_ == 2)                                                        \
             K<2><<<nb_, BLOCK, 0, stream>>>(D);                                    \
@@ -2603,7 +2767,9 @@ void DFSPH::sweep_init_l(bool dens, bool fact, bool div) {
 
 void DFSPH::sweep_init(bool dens, bool fact, bool div) {
     if (!tuned_ && have_lists_) tune_lanes();
-    if (lpp_ == 4)
+    if (lpp_ == ORDERED_LANES)
+        sweep_init_l<ORDERED_LANES>(dens, fact, div);
+    else if (lpp_ == 4)
         sweep_init_l<4>(dens, fact, div);
     else if (lpp_ == 2)
         sweep_init_l<2>(dens, fact, div);
@@ -2615,21 +2781,15 @@ void DFSPH::sweep_init(bool dens, bool fact, bool div) {
 template <bool PRESSURE, bool JACOBI>
 static void launch_sweep(int lanes, unsigned n, hipStream_t s, const Dev &D, int check_done) {
     const unsigned nb = nblocks((size_t)n * lanes);
-    if (JACOBI) {
-        if (lanes == 4)
-            k_jacobi<PRESSURE, 4><<<nb, BLOCK, 0, s>>>(D, check_done);
-        else if (lanes == 2)
-            k_jacobi<PRESSURE, 2><<<nb, BLOCK, 0, s>>>(D, check_done);
-        else
-            k_jacobi<PRESSURE, 1><<<nb, BLOCK, 0, s>>>(D, check_done);
-    } else {
-        if (lanes == 4)
-            k_accel<PRESSURE, 4><<<nb, BLOCK, 0, s>>>(D, check_done);
-        else if (lanes == 2)
-            k_accel<PRESSURE, 2><<<nb, BLOCK, 0, s>>>(D, check_done);
-        else
-            k_accel<PRESSURE, 1><<<nb, BLOCK, 0, s>>>(D, check_done);
+#define SWEEP(L)                                                        \
+    if (lanes == L) {                                                   \
+        if (JACOBI)                                                     \
+            k_jacobi<PRESSURE, L><<<nb, BLOCK, 0, s>>>(D, check_done);  \
+        else                                                            \
+            k_accel<PRESSURE, L><<<nb, BLOCK, 0, s>>>(D, check_done);   \
     }
+    SWEEP(1) SWEEP(2) SWEEP(4) SWEEP(ORDERED_LANES)
+#undef SWEEP
     SPH_HIP(hipGetLastError());
 }
 
@@ -2670,16 +2830,22 @@ void DFSPH::iteration_any(bool force) {
 // One Jacobi iteration of many scenes: three launches in all (see kb_accel).
 void launch_batch_iteration(bool pressure, int lanesA, int lanesJ, const Dev *Ds, const uint4 *bmapA, unsigned nbA,
                             const uint4 *bmapJ, unsigned nbJ, unsigned nscenes, hipStream_t s) {
-#define KB(K, P, L, nb, map) K<P, L><<<nb, BLOCK, 0, s>>>(Ds, map, 1)
-    if (pressure) {
-        if (lanesA == 4) KB(kb_accel, true, 4, nbA, bmapA); else if (lanesA == 2) KB(kb_accel, true, 2, nbA, bmapA); else KB(kb_accel, true, 1, nbA, bmapA);
-        if (lanesJ == 4) KB(kb_jacobi, true, 4, nbJ, bmapJ); else if (lanesJ == 2) KB(kb_jacobi, true, 2, nbJ, bmapJ); else KB(kb_jacobi, true, 1, nbJ, bmapJ);
-        kb_jacobi_reduce<true><<<nscenes, RBLOCK, 0, s>>>(Ds, lanesJ, 1);
-    } else {
-        if (lanesA == 4) KB(kb_accel, false, 4, nbA, bmapA); else if (lanesA == 2) KB(kb_accel, false, 2, nbA, bmapA); else KB(kb_accel, false, 1, nbA, bmapA);
-        if (lanesJ == 4) KB(kb_jacobi, false, 4, nbJ, bmapJ); else if (lanesJ == 2) KB(kb_jacobi, false, 2, nbJ, bmapJ); else KB(kb_jacobi, false, 1, nbJ, bmapJ);
-        kb_jacobi_reduce<false><<<nscenes, RBLOCK, 0, s>>>(Ds, lanesJ, 1);
+#define KB(K, LN, L, nb, map)                                      \
+    if (LN == L) {                                                 \
+        if (pressure)                                              \
+            K<true, L><<<nb, BLOCK, 0, s>>>(Ds, map, 1);           \
+        else                                                       \
+            K<false, L><<<nb, BLOCK, 0, s>>>(Ds, map, 1);          \
     }
+#define KBL(K, LN, nb, map) \
+    KB(K, LN, 1, nb, map) KB(K, LN, 2, nb, map) KB(K, LN, 4, nb, map) KB(K, LN, ORDERED_LANES, nb, map)
+    KBL(kb_accel, lanesA, nbA, bmapA)
+    KBL(kb_jacobi, lanesJ, nbJ, bmapJ)
+    if (pressure)
+        kb_jacobi_reduce<true><<<nscenes, RBLOCK, 0, s>>>(Ds, lanesJ, 1);
+    else
+        kb_jacobi_reduce<false><<<nscenes, RBLOCK, 0, s>>>(Ds, lanesJ, 1);
+#undef KBL
 #undef KB
     SPH_HIP(hipGetLastError());
 }
@@ -2720,7 +2886,8 @@ void DFSPH::pressure_iteration(bool force) { iteration_any<true>(force); }
 // between solves.
 void DFSPH::tune_lanes() {
     tuned_ = true;
-    if (n_ < 65536 || lpp_fixed_) return;
+    if (n_ < SMALL_PARTICLES || lpp_fixed_) return;
+    timed_ = true;
     Dev D = dev();
     fill_u32(stream, reinterpret_cast<unsigned *>(p2_.get()), n_, 0x3f800000u);  // 1.0f
     k_unit_w<<<nblocks(n_), BLOCK, 0, stream>>>(x_.get(), x2_.get(), (unsigned)n_);
@@ -2773,6 +2940,7 @@ void DFSPH::set_lanes_per_particle(int lpp) {
     lpp_ = lpp ? lpp : 1;
     lppA_ = lpp_;
     tuned_ = lpp_fixed_;
+    timed_ = false;
 }
 
 void DFSPH::div_finish(bool scale_pv) {
@@ -2974,9 +3142,9 @@ bool DFSPH::learned_start(bool pressure) {
         else
             REDUCE("learn_scale", k_kref_reduce<false>, D, nblocks(n_));
         if (pressure)
-            LAUNCH("learn_features", k_features<true>, D);
+            LAUNCH_SEQ("learn_features", k_features, true);
         else
-            LAUNCH("learn_features", k_features<false>, D);
+            LAUNCH_SEQ("learn_features", k_features, false);
     }
     if (!use) return false;
     engaged_[solver] = true;
@@ -2992,17 +3160,17 @@ bool DFSPH::learned_start(bool pressure) {
             LAUNCH("learn_start", (k_pred_start<true, true>), D);
         else
             LAUNCH("learn_start", (k_pred_start<true, false>), D);
-        LAUNCH("learn_accel2", k_accel2<true>, D);
-        LAUNCH("learn_jacobi2", k_jacobi2<true>, D);
-        REDUCE("jacobi_reduce", (k_jacobi_reduce<true, true>), D, nblocks(n_), 0);
+        LAUNCH_SEQ("learn_accel2", k_accel2, true);
+        LAUNCH_SEQ("learn_jacobi2", k_jacobi2, true);
+        REDUCE("jacobi_reduce", (k_jacobi_reduce<true, true>), D, nblocks((size_t)n_ * seq_lanes()), 0);
     } else {
         if (mode == 2)
             LAUNCH("learn_start", (k_pred_start<false, true>), D);
         else
             LAUNCH("learn_start", (k_pred_start<false, false>), D);
-        LAUNCH("learn_accel2", k_accel2<false>, D);
-        LAUNCH("learn_jacobi2", k_jacobi2<false>, D);
-        REDUCE("jacobi_reduce", (k_jacobi_reduce<false, true>), D, nblocks(n_), 0);
+        LAUNCH_SEQ("learn_accel2", k_accel2, false);
+        LAUNCH_SEQ("learn_jacobi2", k_jacobi2, false);
+        REDUCE("jacobi_reduce", (k_jacobi_reduce<false, true>), D, nblocks((size_t)n_ * seq_lanes()), 0);
     }
     return true;
 }

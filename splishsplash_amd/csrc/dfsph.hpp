@@ -116,6 +116,10 @@ struct EmitterDesc {
     unsigned counter = 0;  // m_emitCounter
 };
 
+// Below this many particles the lanes per particle follow a rule instead of
+// timings (see DFSPH::tune_lanes).
+constexpr size_t SMALL_PARTICLES = 65536;
+
 class DFSPH;
 // Steps the scenes n_steps times together (batch.hip): their solves run as
 // batched launches (replayed from captured HIP graphs when `graphs`), the
@@ -188,6 +192,8 @@ public:
     void ensure_tuned() {
         if (!tuned_) tune_lanes();
     }
+    // Particles of all scenes stepped together with this one (0: alone).
+    void set_company(size_t n) { company_ = n; }
     int lanes_accel() const { return lppA_; }
     int lanes_jacobi() const { return lpp_; }
     Dev device_state() const { return dev(); }
@@ -366,8 +372,10 @@ private:
     void iteration_any(bool force);
     void tune_lanes();
     int lpp_ = 1;              // lanes per particle of the Jacobi update and the other sweeps
+    int seq_lanes() const { return lpp_ > 4 ? lpp_ : 1; }  // of the sweeps that are not timed (plain sequential sums)
     int lppA_ = 1;             // lanes per particle of the acceleration sweeps (iterations, finish)
-    bool tuned_ = false, lpp_fixed_ = false;
+    size_t company_ = 0;
+    bool tuned_ = false, timed_ = false, lpp_fixed_ = false;  // timed_: lpp_ and lppA_ come from timings
 
 public:
     float tune_ms_[2][3] = {};  // acceleration / Jacobi sweep time at 1, 2, 4 lanes per particle

@@ -309,6 +309,18 @@ int sph_dfsph_step_batch(sph_dfsph_t *handles, size_t n, int n_steps, int thread
             DCHK(handles[k]);
             SPH_REQUIRE(seen.insert(handles[k]).second, SPH_ERR_INVALID, "a handle appears twice in the batch");
         }
+        struct Company {  // tells every scene how many particles step together
+            sph_dfsph_t *h;
+            size_t n;
+            Company(sph_dfsph_t *hh, size_t nn) : h(hh), n(nn) {
+                size_t total = 0;
+                for (size_t k = 0; k < n; k++) total += h[k]->s->n();
+                for (size_t k = 0; k < n; k++) h[k]->s->set_company(total);
+            }
+            ~Company() {
+                for (size_t k = 0; k < n; k++) h[k]->s->set_company(0);
+            }
+        } company(handles, n);
         // A first step that times the sweeps for the lanes per particle runs
         // here for every handle, one handle at a time, before host threads
         // or batched solves take over: lane tuning runs with one handle

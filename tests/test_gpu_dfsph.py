@@ -153,6 +153,35 @@ def test_solver_sweeps_with_split_neighbour_sums(lanes):
     assert g.counters()["lanes_per_particle"] == lanes
 
 
+@pytest.mark.parametrize("side", [3, 11, 26])
+@pytest.mark.parametrize("kw", [{}, {"viscosity_method": 1, "viscosity": 0.05}, {"viscosity_method": 6}])
+def test_shared_pairs_sum_as_one_lane(side, kw):
+    # For small counts 16 lanes evaluate a particle's pairs and its sums
+    # are taken in list order: bit for bit the fields of one lane per
+    # particle, over whole steps with walls, XSPH and both viscosities. A
+    # block of 27 particles has fewer neighbours than lanes; compressed to
+    # 0.75 of its spacing a particle has more than one round of 64.
+    sc = scenes.dam_break_small(per_side=side, **kw)
+    x = (sc["x"] - 0.05) * (0.75 if side == 11 else 1.0)
+    v, p, pv = perturbed_state(x, seed=side)
+    sims = []
+    for lanes in (0, 1):
+        g = capi.TimeStepDFSPH(sc["params"])
+        g.set_fluid(x, v)
+        g.add_boundary_particles(sc["boundary_x"])
+        g.set_lanes_per_particle(lanes)
+        g.init()
+        g.set("p / rho^2", p)
+        g.set("p_v / rho^2", pv)
+        g.step(1 if side == 11 else 3)  # (the compressed block bursts)
+        sims.append(g)
+    assert sims[0].counters()["lanes_per_particle"] == 16 and sims[1].counters()["lanes_per_particle"] == 1
+    if side == 11:
+        assert sims[0].get("fluid neighbor count").max() > 64
+    for f in ("position", "velocity", "density", "factor", "p / rho^2", "p_v / rho^2", "pressure acceleration"):
+        np.testing.assert_array_equal(sims[0].get(f), sims[1].get(f), err_msg=f)
+
+
 def vm_scene(n=16, corner=0.06):
     x = scenes.lattice_block((n, n, n), 0.05, (corner, corner, corner), jitter=0.002, seed=5)
     # three particles inside the wall (projected back by the volume-map stage)

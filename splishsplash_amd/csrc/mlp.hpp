@@ -24,10 +24,17 @@ void mlp_forward(hipStream_t s, const float *theta, const float *x, unsigned n, 
 class MLPTrainer {
 public:
     DBuf<float> partial, grad, loss_part, adam_m, adam_v, loss;
-    unsigned waves = 0;
+    DBuf<short> packed;  // BF16 weights in operand order (see mlp.hip)
+    unsigned parts = 0;
     void loss_grad(hipStream_t s, const float *theta, const float *x, const float *t, unsigned n);
-    // One Adam step on theta with the gradient of the last loss_grad.
-    void adam(hipStream_t s, float *theta, int step, float lr);
+    // Adam from zero moments: start, then step 1, 2, ... on minibatches of n
+    // rows; theta changes only through step in between.
+    void start(hipStream_t s, const float *theta);
+    void step(hipStream_t s, float *theta, const float *x, const float *t, unsigned n, int step, float lr);
+
+private:
+    void pack(hipStream_t s, const float *theta);
+    void sums(hipStream_t s, const float *theta, const float *x, const float *t, unsigned n);
 };
 
 }  // namespace sph

@@ -63,3 +63,24 @@ def test_training_fits_a_smooth_target():
     assert l1 < 0.05 * l0, (l0, l1)
     yo, _ = M.forward(th.astype(np.float64), x)
     assert float(np.mean((yo - t) ** 2)) < 0.1 * l0
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 127, 129, 32768, 32801])
+def test_gradient_at_tile_and_block_edges(n):
+    # tiles of 32 rows, four waves a block, at most 256 blocks: partial
+    # tiles, waves and blocks without a tile, and a second round of tiles.
+    # BF16 weights, activations and their gradients (2^-9 each) in FP32 sums:
+    # the bound of test_gradient_matches_oracle.
+    rng = np.random.default_rng(n)
+    theta = M.init(4).astype(np.float32)
+    x = rng.normal(size=(n, 6)).astype(np.float32)
+    t = rng.normal(size=n).astype(np.float32)
+    loss, g = capi.mlp_loss_grad(theta, x, t)
+    lo, go = M.loss_and_grad(theta.astype(np.float64), x.astype(np.float64), t)
+    assert loss == pytest.approx(lo, rel=3e-2)
+    assert rel(g, go) < 5e-2
+    assert g @ go / (np.linalg.norm(g) * np.linalg.norm(go)) > 0.999
+    # no steps: the shuffled rows give the same loss
+    th, l0 = capi.mlp_train(theta, x, t, steps=0, batch=7, seed=3)
+    np.testing.assert_array_equal(th, theta)
+    assert l0 == pytest.approx(loss, rel=1e-5)

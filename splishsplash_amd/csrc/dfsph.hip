@@ -891,6 +891,50 @@ __global__ __launch_bounds__(BLOCK) void k_mrho_to_w(Dev D) {
     reinterpret_cast<float *>(D.x + i)[3] = mass_of(D, i) / D.rho[i];
 }
 
+// Field access in particle-id order: out[id[k]] = component values of slot k
+// (COMPS 3: x, y, z; 1: component w of a float4), and back. The scattered
+// side stays on the device, where a particle's slot and id are close to each
+// other in cache; the host moves one contiguous block.
+template <int COMPS>
+__global__ __launch_bounds__(BLOCK) void k_field_out4(const float4 *__restrict__ f, const unsigned *__restrict__ id,
+                                                      unsigned n, float *__restrict__ out) {
+    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const float4 v = f[k];
+    const size_t o = id[k];
+    if (COMPS == 3) {
+        out[3 * o] = v.x;
+        out[3 * o + 1] = v.y;
+        out[3 * o + 2] = v.z;
+    } else {
+        out[o] = v.w;
+    }
+}
+__global__ __launch_bounds__(BLOCK) void k_field_out1(const unsigned *__restrict__ f, const unsigned *__restrict__ id,
+                                                      unsigned n, unsigned *__restrict__ out) {
+    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) out[id[k]] = f[k];
+}
+// f[k] = (in[id[k]], 0); zero (may be null) is cleared beside it.
+__global__ __launch_bounds__(BLOCK) void k_field_in4(const float *__restrict__ in, const unsigned *__restrict__ id,
+                                                     unsigned n, float4 *__restrict__ f, float4 *__restrict__ zero) {
+    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const size_t o = id[k];
+    f[k] = make_float4(in[3 * o], in[3 * o + 1], in[3 * o + 2], 0.f);
+    if (zero) zero[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+__global__ __launch_bounds__(BLOCK) void k_field_in1(const unsigned *__restrict__ in, const unsigned *__restrict__ id,
+                                                     unsigned n, unsigned *__restrict__ f) {
+    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) f[k] = in[id[k]];
+}
+
+__global__ void k_set_time(Ctl *C, double t, double h) {
+    C->time = t;
+    C->h = h;
+}
+
 // Tuning input: positions with a unit stiffness in w.
 __global__ __launch_bounds__(BLOCK) void k_unit_w(const float4 *__restrict__ x, float4 *__restrict__ y, unsigned n) {
     const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -3648,36 +3692,24 @@ void DFSPH::get_field(const std::string &name, void *host, size_t bytes) {
     else if (name == "boundary neighbor count") u1 = cb_.get();
     else throw Error(SPH_ERR_NOTFOUND, "unknown field '" + name + "'");
     SPH_REQUIRE(bytes == n * comps * 4, SPH_ERR_INVALID, "size mismatch for field '" + name + "'");
-    const std::vector<unsigned> id = ids_host();
-    if (f4) {
-        std::vector<float4> t(n);
-        SPH_HIP(hipMemcpy(t.data(), f4, n * sizeof(float4), hipMemcpyDeviceToHost));
-        float *out = static_cast<float *>(host);
-        for (size_t s = 0; s < n; s++) {
-            const size_t k = id[s];
-            if (vmpart == 2) {
-                out[k] = t[s].w;
-            } else {
-                out[3 * k] = t[s].x;
-                out[3 * k + 1] = t[s].y;
-                out[3 * k + 2] = t[s].z;
-            }
-        }
-    } else if (f1) {
-        std::vector<float> t(n);
-        SPH_HIP(hipMemcpy(t.data(), f1, n * sizeof(float), hipMemcpyDeviceToHost));
-        float *out = static_cast<float *>(host);
-        for (size_t s = 0; s < n; s++) out[id[s]] = t[s];
-    } else {
-        std::vector<unsigned> t(n);
-        if ((name == "boundary neighbor count" && !(P.boundary_handling_method == SPH_BOUNDARY_AKINCI2012 && nb_ > 0)) ||
-            (name == "state" && !states_))
-            std::fill(t.begin(), t.end(), 0u);
-        else
-            SPH_HIP(hipMemcpy(t.data(), u1, n * sizeof(unsigned), hipMemcpyDeviceToHost));
-        unsigned *out = static_cast<unsigned *>(host);
-        for (size_t s = 0; s < n; s++) out[id[s]] = t[s];
+    if (n == 0) return;
+    if ((name == "boundary neighbor count" && !(P.boundary_handling_method == SPH_BOUNDARY_AKINCI2012 && nb_ > 0)) ||
+        (name == "state" && !states_)) {
+        std::memset(host, 0, bytes);
+        return;
     }
+    io_.reserve(3 * (size_t)stride_);
+    const unsigned nn = (unsigned)n;
+    if (f4 && vmpart != 2)
+        k_field_out4<3><<<nblocks(n), BLOCK, 0, stream>>>(f4, id_.get(), nn, io_.get());
+    else if (f4)
+        k_field_out4<1><<<nblocks(n), BLOCK, 0, stream>>>(f4, id_.get(), nn, io_.get());
+    else
+        k_field_out1<<<nblocks(n), BLOCK, 0, stream>>>(f1 ? reinterpret_cast<const unsigned *>(f1) : u1, id_.get(), nn,
+                                                       reinterpret_cast<unsigned *>(io_.get()));
+    SPH_HIP(hipGetLastError());
+    SPH_HIP(hipMemcpyAsync(host, io_.get(), bytes, hipMemcpyDeviceToHost, stream));
+    SPH_HIP(hipStreamSynchronize(stream));
 }
 
 void DFSPH::set_field(const std::string &name, const void *host, size_t bytes) {
@@ -3699,37 +3731,24 @@ void DFSPH::set_field(const std::string &name, const void *host, size_t bytes) {
     else if (name == "p_v / rho^2") f1 = pv_.get();
     else if (name != "state") throw Error(SPH_ERR_NOTFOUND, "unknown or read-only field '" + name + "'");
     SPH_REQUIRE(bytes == n * comps * 4, SPH_ERR_INVALID, "size mismatch for field '" + name + "'");
-    const std::vector<unsigned> id = ids_host();
     if (name == "state") {
         // ParticleState: 0 active, 1 animated by an emitter, 2 fixed
         const unsigned *in = static_cast<const unsigned *>(host);
-        std::vector<unsigned> t(n);
-        for (size_t s = 0; s < n; s++) {
-            t[s] = in[id[s]];
-            SPH_REQUIRE(t[s] <= 2u, SPH_ERR_INVALID, "particle state must be 0, 1 or 2");
-        }
+        for (size_t k = 0; k < n; k++) SPH_REQUIRE(in[k] <= 2u, SPH_ERR_INVALID, "particle state must be 0, 1 or 2");
         enable_states();
-        SPH_HIP(hipStreamSynchronize(stream));
-        SPH_HIP(hipMemcpy(pst_.get(), t.data(), n * sizeof(unsigned), hipMemcpyHostToDevice));
-        return;
     }
-    const float *in = static_cast<const float *>(host);
-    if (f4) {
-        std::vector<float4> t(n);
-        for (size_t s = 0; s < n; s++) {
-            const size_t k = id[s];
-            t[s] = make_float4(in[3 * k], in[3 * k + 1], in[3 * k + 2], 0.f);
-        }
-        SPH_HIP(hipMemcpy(f4, t.data(), n * sizeof(float4), hipMemcpyHostToDevice));
-        if (name == "position") {
-            std::vector<float4> z(n, make_float4(0.f, 0.f, 0.f, 0.f));
-            SPH_HIP(hipMemcpy(xc_.get(), z.data(), n * sizeof(float4), hipMemcpyHostToDevice));
-        }
-    } else {
-        std::vector<float> t(n);
-        for (size_t s = 0; s < n; s++) t[s] = in[id[s]];
-        SPH_HIP(hipMemcpy(f1, t.data(), n * sizeof(float), hipMemcpyHostToDevice));
-    }
+    if (n == 0) return;
+    io_.reserve(3 * (size_t)stride_);
+    const unsigned nn = (unsigned)n;
+    SPH_HIP(hipMemcpyAsync(io_.get(), host, bytes, hipMemcpyHostToDevice, stream));
+    if (f4)
+        k_field_in4<<<nblocks(n), BLOCK, 0, stream>>>(io_.get(), id_.get(), nn, f4,
+                                                      name == "position" ? xc_.get() : nullptr);
+    else
+        k_field_in1<<<nblocks(n), BLOCK, 0, stream>>>(reinterpret_cast<const unsigned *>(io_.get()), id_.get(), nn,
+                                                      f1 ? reinterpret_cast<unsigned *>(f1) : pst_.get());
+    SPH_HIP(hipGetLastError());
+    SPH_HIP(hipStreamSynchronize(stream));
 }
 
 void DFSPH::get_neighbors(int boundary, unsigned *offsets, unsigned *indices, size_t capacity, size_t *nnz) {
@@ -3803,8 +3822,8 @@ void DFSPH::counters(sph_dfsph_counters_t *c) {
 void DFSPH::set_time(double t, double h) {
     SPH_REQUIRE(h > 0, SPH_ERR_INVALID, "time step size must be > 0");
     // h_step is taken from h by the next neighbourhood search
-    upload_ctl_field(offsetof(Ctl, h), &h, sizeof(double));
-    upload_ctl_field(offsetof(Ctl, time), &t, sizeof(double));
+    k_set_time<<<1, 1, 0, stream>>>(ctl_.get(), t, h);
+    SPH_HIP(hipGetLastError());
 }
 
 void DFSPH::sync() { SPH_HIP(hipStreamSynchronize(stream)); }

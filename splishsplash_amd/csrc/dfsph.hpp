@@ -298,6 +298,7 @@ private:
     DBuf<float4> minv_, cgx_, cgr_, cgp_, cgz_, cgt_;
     DBuf<double> partial_;
     DBuf<Ctl> ctl_;
+    DBuf<float> io_;       // field values in id order, on their way from or to the host
     Ctl *hctl_ = nullptr;  // pinned mirror
     CellSorter fsort_, bsort_;
     long long totIt_ = 0, totItV_ = 0, totVisco_ = 0;

@@ -109,6 +109,12 @@ __device__ inline unsigned xcd_block() {
     return xcd < rem ? xcd * (per + 1u) + local : rem * (per + 1u) + (xcd - rem) * per + local;
 }
 
+// Its inverse: the hardware block id of a grid of B that works on block q.
+__device__ inline unsigned xcd_slot(unsigned q, unsigned B) {
+    const unsigned per = B / 8u, rem = B % 8u, head = rem * (per + 1u);
+    return q < head ? q % (per + 1u) * 8u + q / (per + 1u) : (q - head) % per * 8u + rem + (q - head) / per;
+}
+
 // ------------------------------------------------------------ gathers
 // Neighbour-side reads of a float4 array through a buffer resource: the
 // element's 32-bit byte offset (one shift) replaces 64-bit address

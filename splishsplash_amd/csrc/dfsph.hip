@@ -136,6 +136,216 @@ __device__ __forceinline__ void fluid_pairs(const Dev &D, unsigned i, unsigned h
     }
 }
 
+// ---------------------------------------------------------------- tiles
+// The sweeps of the solver iterations visit the same lists some forty times a
+// step, and the gathers bound them: a wave's 64 neighbours lie in 42-46
+// cache lines, which the vector cache looks up one per cycle (texture data
+// path 75 % busy in k_accel, 90 % in k_jacobi at 1M particles, whatever the
+// arithmetic between: 12 % fewer vector instructions left the times as they
+// were). Consecutive particles share most of their neighbours, so a tile of
+// 256 needs about 8 slots a particle instead of 30: a tiled sweep copies
+// those to LDS once, coalesced, and its pairs read LDS. At 1M particles
+// (pressure / divergence iterations) k_accel 47 / 44 -> 28 / 36 us, k_jacobi
+// 73 / 65 -> 52 / 47 us; at 69k 9.3 / 10.0 -> 8.1 / 9.6 and 14.8 / 14.0 ->
+// 12.2 / 11.4 us. They are now bound by the vector instructions, 45 a pair,
+// some 12 % of them in the FP64 band of table_step. Tiles of 128 particles
+// take as long in the sweeps and half as long again to build.
+//
+// k_tile_lists, once a step: marks the tile's neighbour slots in a bitmap of
+// the 65536 slots around the tile, numbers the marked ones in slot order and
+// rewrites the packed lists with these numbers, entries in the same order
+// (86 us at 1M particles, 31 us at 69k; bound by LDS: a marked slot is an
+// atomic, a rewritten one two reads).
+// A tile with more than TILE_CAP slots, or slots outside the window, keeps a
+// count of zero and its sweeps read memory as before.
+constexpr unsigned TILE_WORDS = 65536 / 32;
+__global__ __launch_bounds__(TILE) void k_tile_lists(Dev D, uint4 *__restrict__ nt16,
+                                                     unsigned *__restrict__ tslot, unsigned *__restrict__ tcount) {
+    __shared__ __align__(16) unsigned bits[TILE_WORDS], first[TILE_WORDS];
+    __shared__ unsigned wtot[TILE / 64], bad;
+    constexpr unsigned PER = TILE_WORDS / TILE;
+    const unsigned t = threadIdx.x, lane = t & 63u, blk = xcd_block();
+    const unsigned i0 = blk * TILE, i = i0 + t;
+#pragma unroll
+    for (unsigned q = 0; q < PER; q++) bits[q * TILE + t] = 0u;
+    if (t == 0) bad = 0u;
+    __syncthreads();
+    const unsigned cnt = i < D.n ? D.cf[i] : 0u, nw = (cnt + 1u) >> 1;
+    const unsigned *__restrict__ P = D.nf16 + i;
+    const size_t S = D.stride;
+    // place of entry d (a slot less i) in the window
+    auto place = [&](int d) { return (unsigned)(d + (int)t + 32768); };
+    bool far = false;
+    auto mark = [&](unsigned p) {
+        if (p < 65536u)
+            atomicOr(&bits[p >> 5], 1u << (p & 31u));
+        else
+            far = true;
+    };
+    auto quad = [&](unsigned w, unsigned *a) {
+#pragma unroll
+        for (unsigned q = 0; q < 4u; q++) a[q] = P[(w + q < nw ? w + q : w) * S];
+    };
+    for (unsigned w = 0; w < nw; w += 4u) {
+        unsigned a[4];
+        quad(w, a);
+#pragma unroll
+        for (unsigned q = 0; q < 4u; q++) {
+            if (2u * (w + q) < cnt) mark(place((int)(short)(a[q] & 0xffffu)));
+            if (2u * (w + q) + 1u < cnt) mark(place((int)a[q] >> 16));
+        }
+    }
+    if (far) bad = 1u;
+    __syncthreads();
+    // thread t numbers words t PER .. t PER + PER - 1
+    unsigned b[PER], sum = 0;
+#pragma unroll
+    for (unsigned q = 0; q < PER; q++) {
+        b[q] = bits[t * PER + q];
+        sum += (unsigned)__popc(b[q]);
+    }
+    unsigned inc = sum;
+    for (unsigned o = 1; o < 64u; o <<= 1) {
+        const unsigned v = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += v;
+    }
+    if (lane == 63u) wtot[t >> 6] = inc;
+    __syncthreads();
+    unsigned base = inc - sum, total = 0;
+#pragma unroll
+    for (unsigned q = 0; q < TILE / 64; q++) {
+        if (q < (t >> 6)) base += wtot[q];
+        total += wtot[q];
+    }
+    const bool fits = total <= TILE_CAP && bad == 0u;
+    if (t == 0) tcount[blk] = fits ? total : 0u;
+    if (!fits) return;
+    short *const out = reinterpret_cast<short *>(tslot + (size_t)blk * (TILE_CAP / 2));
+#pragma unroll
+    for (unsigned q = 0; q < PER; q++) {
+        first[t * PER + q] = base;
+        for (unsigned m = b[q]; m != 0u; m &= m - 1u) {
+            const short d = (short)((int)(t * PER + q) * 32 + __ffs(m) - 1 - 32768);
+            out[base] = d;
+            // an odd count fills its last word with the same slot
+            if (++base == total && (total & 1u)) out[base] = d;
+        }
+    }
+    __syncthreads();
+    auto number = [&](unsigned p) {
+        return first[p >> 5] + (unsigned)__popc(bits[p >> 5] & ((1u << (p & 31u)) - 1u));
+    };
+    for (unsigned w = 0; w < nw; w += 4u) {
+        unsigned a[4];
+        quad(w, a);
+#pragma unroll
+        for (unsigned q = 0; q < 4u; q++) {
+            const unsigned lo = 2u * (w + q) < cnt ? number(place((int)(short)(a[q] & 0xffffu))) : 0u;
+            const unsigned hi = 2u * (w + q) + 1u < cnt ? number(place((int)a[q] >> 16)) : 0u;
+            a[q] = lo | (hi << 16);
+        }
+        nt16[(w >> 2) * S + i] = make_uint4(a[0], a[2], a[1], a[3]);
+    }
+}
+
+// Copies the `cnt` slots of tile blk to LDS: put(k, load(slot)) for the k-th
+// slot, by a block of NT threads, the loads of all its slots in flight.
+template <unsigned NT, class LD, class PUT>
+__device__ __forceinline__ void tile_stage(const Dev &D, unsigned blk, unsigned cnt, LD &&load, PUT &&put) {
+    constexpr unsigned R = (TILE_CAP / 2 + NT - 1) / NT;
+    const unsigned *__restrict__ W = D.tslot + (size_t)blk * (TILE_CAP / 2);
+    const unsigned words = (cnt + 1u) >> 1, i0 = blk * TILE;
+    unsigned w[R];
+    decltype(load(0u)) lo[R], hi[R];
+#pragma unroll
+    for (unsigned r = 0; r < R; r++) {
+        const unsigned k = r * NT + threadIdx.x;
+        w[r] = W[k < words ? k : words - 1u];
+    }
+#pragma unroll
+    for (unsigned r = 0; r < R; r++) {
+        if (r * NT >= words) break;
+        lo[r] = load(nb_lo(i0, w[r]));
+        hi[r] = load(nb_hi(i0, w[r]));
+    }
+#pragma unroll
+    for (unsigned r = 0; r < R; r++) {
+        if (r * NT >= words) break;
+        const unsigned k = r * NT + threadIdx.x;
+        if (k < words) {
+            put(2u * k, lo[r]);
+            put(2u * k + 1u, hi[r]);
+        }
+    }
+}
+
+// fluid_pairs of a tile: the same split and order, f(LDS places...) for four,
+// two or one neighbours. A sweep from LDS would wait for its list words
+// (each a trip to HBM) instead of its gathers, so the lane loads them by the
+// quad (its 4 / LPP words) and holds two or three quads in registers: the
+// first are loaded before the tile is staged. (Words loaded where they are
+// used: k_accel 43 / 51 us, k_jacobi 61 / 58 us at 1M particles.)
+template <int LPP> struct TileWords {
+    static constexpr int W = 4 / LPP;  // words of a quad per lane
+    typedef unsigned Quad __attribute__((ext_vector_type(W == 1 ? 2 : W)));  // (one word: .x)
+    Quad c, n, m;
+    const unsigned *P;
+    __device__ __forceinline__ static Quad load(const unsigned *p) {
+        if constexpr (W == 1)
+            return Quad{*p, 0u};
+        else
+            return *reinterpret_cast<const Quad *>(p);
+    }
+    __device__ __forceinline__ TileWords(const Dev &D, unsigned i, unsigned hl)
+        : P(D.nt16 + 4 * (size_t)i + (LPP == 4 ? ((hl & 1u) << 1 | hl >> 1) : W * hl)) {
+        const size_t S = 4 * (size_t)D.stride;
+        const unsigned last = D.quads16 - 1u;
+        const bool act = i < D.n;
+        c = act ? load(P) : Quad{};
+        n = act ? load(P + (last < 1u ? last : 1u) * S) : Quad{};
+        m = act && W < 4 ? load(P + (last < 2u ? last : 2u) * S) : Quad{};
+    }
+    template <class F> __device__ __forceinline__ void pairs(const Dev &D, unsigned hl, unsigned cnt, F &&f) {
+        constexpr unsigned AHEAD = W < 4 ? 3 : 2;
+        const size_t S = 4 * (size_t)D.stride;
+        const unsigned full = cnt >> 1, quads = (cnt + 7u) >> 3;  // words of two neighbours; quads
+        const unsigned *p = P + AHEAD * S;
+        unsigned w = hl, k = AHEAD;
+        auto four = [&](unsigned a, unsigned b) { f(a & 0xffffu, a >> 16, b & 0xffffu, b >> 16); };
+        auto two = [&](unsigned a) { f(a & 0xffffu, a >> 16); };
+        for (; w + (W - 1) * LPP < full; w += 4, k++, p += S) {
+            const Quad q = c;
+            c = n;
+            if (W < 4) n = m;
+            if (k < quads) (W < 4 ? m : n) = load(p);
+            if constexpr (W == 4) {
+                four(q.x, q[2]);
+                four(q.y, q[3]);
+            } else if constexpr (W == 2) {
+                four(q.x, q.y);
+            } else {
+                two(q.x);
+            }
+        }
+        // the lane's rest of c: fewer than W full words, and the odd entry
+        unsigned a = c.x;
+        if constexpr (W == 4)
+            if (w + 1 < full) {
+                four(c.x, c[2]);
+                a = c.y;
+                c[2] = c[3];
+                w += 2;
+            }
+        if constexpr (W > 1)
+            if (w < full) {
+                two(a);
+                a = c[W / 2];
+                w += LPP;
+            }
+        if ((cnt & 1u) && w == full) f(a & 0xffffu);
+    }
+};
+
 // Calls f(xb) for the Akinci boundary neighbours of particle i in order.
 template <class F>
 __device__ __forceinline__ void akinci_pairs(const Dev &D, unsigned i, unsigned cb, F &&f) {
@@ -535,7 +745,7 @@ __global__ __launch_bounds__(BLOCK) void k_sweep_init(Dev D) {
 // t = (c, r) with a_i += c r; false where the pair carries no pressure.
 __device__ __forceinline__ bool accel_term(const Dev &D, const float4 &xi, float pi, const float4 &xj, float inv_rho0i,
                                            float *t) {
-    const float ps = D.model ? pi + xj.w * inv_rho0i : pi + xj.w;
+    const float ps = pi + xj.w * inv_rho0i;  // (times 1 with a single model)
     if (!(fabsf(ps) > D.eps)) return false;
     float3 r;
     const float g = kernel_G(xi, xj, D.K, r);
@@ -574,8 +784,28 @@ __device__ __forceinline__ void accel_maps(const Dev &D, unsigned i, const float
     acc = make_float3(ax, ay, az);
 }
 
-// Pressure acceleration of particle i (zero unless live), complete in lane
-// hl == 0. The lanes of a particle call this together.
+// Pressure acceleration of particle i from its lanes' fluid sums acc,
+// complete in lane hl == 0. The lanes of a particle call this together.
+template <int LPP>
+__device__ __forceinline__ float3 accel_total(const Dev &D, unsigned i, unsigned hl, bool live, const float4 &xi,
+                                              float pi, float *acc, float *__restrict__ T) {
+    lanes_join<LPP, SumVec>(acc);
+    if (D.bmode == 1)
+        akinci_sums<LPP, SumAdd<3>>(D, i, hl, live && fabsf(pi) > D.eps ? D.cb[i] : 0u, T, acc,
+                                    [&](const float4 &xb, float *t) {
+                                        float3 r;
+                                        const float g = kernel_G(xi, xb, D.K, r);
+                                        t[0] = pi * (-xb.w * (g * r.x));
+                                        t[1] = pi * (-xb.w * (g * r.y));
+                                        t[2] = pi * (-xb.w * (g * r.z));
+                                        return true;
+                                    });
+    float3 a = make_float3(acc[0], acc[1], acc[2]);
+    if (live && hl == 0) accel_maps(D, i, xi, pi, a);
+    return a;
+}
+
+// The same with the fluid sums: zero unless live.
 template <int LPP>
 __device__ __forceinline__ float3 particle_accel(const Dev &D, unsigned i, unsigned hl, bool live,
                                                  const float *__restrict__ P, float *__restrict__ T) {
@@ -591,20 +821,7 @@ __device__ __forceinline__ float3 particle_accel(const Dev &D, unsigned i, unsig
             D, i, hl, D.cf[i], T, acc, loads([&](unsigned j) { return X.all(j); }),
             [&](unsigned, const auto &q, float *t) { return accel_term(D, xi, pi, q.a, ir, t); });
     }
-    lanes_join<LPP, SumVec>(acc);
-    if (D.bmode == 1)
-        akinci_sums<LPP, SumAdd<3>>(D, i, hl, live && fabsf(pi) > D.eps ? D.cb[i] : 0u, T, acc,
-                                    [&](const float4 &xb, float *t) {
-                                        float3 r;
-                                        const float g = kernel_G(xi, xb, D.K, r);
-                                        t[0] = pi * (-xb.w * (g * r.x));
-                                        t[1] = pi * (-xb.w * (g * r.y));
-                                        t[2] = pi * (-xb.w * (g * r.z));
-                                        return true;
-                                    });
-    float3 a = make_float3(acc[0], acc[1], acc[2]);
-    if (live && hl == 0) accel_maps(D, i, xi, pi, a);
-    return a;
+    return accel_total<LPP>(D, i, hl, live, xi, pi, acc, T);
 }
 
 // The acceleration sweep of block `blk` of a particle range; the single
@@ -633,6 +850,41 @@ __global__ __launch_bounds__(BLOCK) void k_accel(Dev D, int check_done) {
     accel_sweep<PRESSURE, LPP>(D, xcd_block(), check_done);
 }
 
+// The same for a tile of one model's particles (TILE LPP threads).
+template <bool PRESSURE, int LPP>
+__global__ __launch_bounds__(TILE *LPP) void k_accel_tile(Dev D, int check_done) {
+    __shared__ float4 tile[TILE_CAP];
+    if (check_done && (PRESSURE ? D.ctl->done : D.ctl->done_v)) return;
+    const unsigned blk = xcd_block(), i = blk * TILE + threadIdx.x / LPP, h = threadIdx.x % LPP;
+    const unsigned m = D.tcount[blk];
+    const bool act = i < D.n;
+    const bool live = act && is_active(D, i);
+    const float4 xi = live ? D.x[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float pi = live ? (PRESSURE ? D.p : D.pv)[i] : 0.f;
+    const unsigned cnt = live ? D.cf[i] : 0u;
+    float acc[3] = {0.f, 0.f, 0.f};
+    const F4Gather X(D.x, D.n);
+    if (m != 0u) {
+        TileWords<LPP> words(D, i, h);
+        tile_stage<TILE * LPP>(
+            D, blk, m, [&](unsigned j) { return X.all(j); }, [&](unsigned k, const float4 &v) { tile[k] = v; });
+        __syncthreads();
+        words.pairs(D, h, cnt, [&](auto... k) {
+            const float4 xj[] = {tile[k]...};
+            float t[SumVec::NT];
+#pragma unroll
+            for (unsigned q = 0; q < sizeof...(k); q++)
+                if (accel_term(D, xi, pi, xj[q], 1.f, t)) sum_terms<SumVec>(t, acc);
+        });
+    } else {
+        fluid_sums<LPP, SumVec>(
+            D, i, h, cnt, nullptr, acc, loads([&](unsigned j) { return X.all(j); }),
+            [&](unsigned, const auto &q, float *t) { return accel_term(D, xi, pi, q.a, 1.f, t); });
+    }
+    const float3 a = accel_total<LPP>(D, i, h, live, xi, pi, acc, nullptr);
+    if (act && h == 0) D.ap[i] = make_float4(a.x, a.y, a.z, 0.f);
+}
+
 // Many scenes in one launch: block b works on particle block bmap[b].y of
 // scene bmap[b].x, whose state Ds[bmap[b].x] describes; bmap[b].z is the
 // partial-sum slot the same particles take in the scene's own launch.
@@ -644,45 +896,44 @@ __global__ __launch_bounds__(BLOCK) void kb_accel(const Dev *__restrict__ Ds, co
 }
 
 // t = (g, d) with s += g d: (a_i - a_j) . gradW_ij = g_ij ((a_i - a_j) . r_ij)
+__device__ __forceinline__ float aij_dot(const float4 &ai, const float4 &aj, const float3 &r) {
+    return fmaf(ai.z - aj.z, r.z, fmaf(ai.y - aj.y, r.y, (ai.x - aj.x) * r.x));
+}
 __device__ __forceinline__ bool aij_term(const float4 &xi, const float4 &ai, const float4 &xj, const float4 &aj,
                                          const KernelConst &K, float *t) {
     float3 r;
     t[0] = kernel_G(xi, xj, K, r);
-    t[1] = fmaf(ai.z - aj.z, r.z, fmaf(ai.y - aj.y, r.y, (ai.x - aj.x) * r.x));
+    t[1] = aij_dot(ai, aj, r);
     return true;
 }
 
 // compute_aij_pj (TimeStepDFSPH.cpp:1370-1420) and the Jacobi update of
 // pressureSolveIteration / divergenceSolveIteration (:544-706), FP64 error
 // sum finished in the last block.
-template <bool PRESSURE, int LPP>
-__device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigned part, int check_done) {
-    __shared__ double lds[BLOCK / 64];
-    __shared__ float plds[PAIR_LDS<LPP, SumDot::NT>];
-    float *const T = pair_part<LPP, SumDot::NT>(plds);
-    Ctl *C = D.ctl;
-    if (check_done && (PRESSURE ? C->done : C->done_v)) return;
-    const unsigned t = blk * blockDim.x + threadIdx.x;
-    const unsigned i = t / LPP, hl = t % LPP;
-    // the pressure update skips particles that are not active
-    // (TimeStepDFSPH.cpp:578-579); the divergence update takes every particle
-    const bool act = i < D.n && (!PRESSURE || is_active(D, i)) && in_solve(D, i);
-    const double h = C->h;
-    double err = 0.0, over = 0.0;
-    float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), ai = xi;
-    unsigned cnt = 0, cb = 0;
-    float s = 0.f;
-    if (act) {
-        xi = D.x[i];
-        ai = D.ap[i];
-        cnt = D.cf[i];
-        const F4Gather X(D.x, D.n), A(D.ap, D.n);
-        fluid_sums<LPP, SumDot>(
-            D, i, hl, cnt, T, &s, loads([&](unsigned j) { return X.xyz(j); }, [&](unsigned j) { return A.xyz(j); }),
-            [&](unsigned, const auto &q, float *u) { return aij_term(xi, ai, q.a, q.b, D.K, u); });
-    }
+// A particle's own values in the update.
+struct JacobiOwn {
+    float alpha, radv, p;
+};
+template <bool PRESSURE> __device__ __forceinline__ JacobiOwn jacobi_own(const Dev &D, unsigned i) {
+    return {D.alpha[i], D.radv[i], (PRESSURE ? D.p : D.pv)[i]};
+}
+// The pressure update skips particles that are not active
+// (TimeStepDFSPH.cpp:578-579); the divergence update takes every particle.
+template <bool PRESSURE> __device__ __forceinline__ bool jacobi_takes(const Dev &D, unsigned i) {
+    return i < D.n && (!PRESSURE || is_active(D, i)) && in_solve(D, i);
+}
+
+// The update of particle i (if act) from its lanes' fluid sums s; own()
+// gives its JacobiOwn; err and over are its shares of the error sums.
+template <bool PRESSURE, int LPP, class OWN>
+__device__ __forceinline__ void jacobi_particle(const Dev &D, unsigned i, unsigned hl, bool act, unsigned cnt,
+                                                const float4 &xi, const float4 &ai, float s, float *__restrict__ T,
+                                                OWN &&own, double &err, double &over) {
+    const double h = D.ctl->h;
+    err = over = 0.0;
     lanes_join<LPP, SumDot>(&s);
     s *= D.V;
+    unsigned cb = 0;
     if (act && D.bmode == 1) cb = D.cb[i];
     if (D.bmode == 1)
         akinci_sums<LPP, SumAdd<1>>(D, i, hl, cb, T, &s, [&](const float4 &xb, float *u) {
@@ -708,12 +959,12 @@ __device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigne
                 s -= (ai.x * gb.x + ai.y * gb.y) + ai.z * gb.z;
             }
         }
-        const float alpha = D.alpha[i];
+        const JacobiOwn o = own();
         if (PRESSURE) {
             const float aij = s * (float)(h * h);
-            const float si = 1.0f - D.radv[i];
+            const float si = 1.0f - o.radv;
             const float res = fminf(si - aij, 0.0f);
-            const float pn = fmaxf(D.p[i] - 0.5f * (si - aij) * alpha, 0.0f);
+            const float pn = fmaxf(o.p - 0.5f * (si - aij) * o.alpha, 0.0f);
             D.p[i] = pn;
             reinterpret_cast<float *>(D.x + i)[3] = stiff_w(D, i, pn);
             const double r0 = rho0_of(D, i);
@@ -721,10 +972,10 @@ __device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigne
             if (pn > 0.0f && si - aij > 0.0f) over = r0 * (double)(si - aij);
         } else {
             const float aij = s * (float)h;
-            const float si = -D.radv[i];
+            const float si = -o.radv;
             float res = fminf(si - aij, 0.0f);
             if (nnb < 20u) res = 0.0f;
-            const float pn = fmaxf(D.pv[i] - 0.5f * (si - aij) * alpha, 0.0f);
+            const float pn = fmaxf(o.p - 0.5f * (si - aij) * o.alpha, 0.0f);
             D.pv[i] = pn;
             reinterpret_cast<float *>(D.x + i)[3] = stiff_w(D, i, pn);
             const double r0 = rho0_of(D, i);
@@ -732,9 +983,112 @@ __device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigne
             if (pn > 0.0f && si - aij > 0.0f && nnb >= 20u) over = r0 * (double)(si - aij);
         }
     }
+}
+
+// The lane's share of the fluid sum, neighbours read from memory.
+template <int LPP>
+__device__ __forceinline__ void aij_sums(const Dev &D, unsigned i, unsigned hl, unsigned cnt, float *__restrict__ T,
+                                         const float4 &xi, const float4 &ai, float *s) {
+    const F4Gather X(D.x, D.n), A(D.ap, D.n);
+    fluid_sums<LPP, SumDot>(
+        D, i, hl, cnt, T, s, loads([&](unsigned j) { return X.xyz(j); }, [&](unsigned j) { return A.xyz(j); }),
+        [&](unsigned, const auto &q, float *u) { return aij_term(xi, ai, q.a, q.b, D.K, u); });
+}
+
+template <bool PRESSURE, int LPP>
+__device__ __forceinline__ void jacobi_sweep(const Dev &D, unsigned blk, unsigned part, int check_done) {
+    __shared__ double lds[BLOCK / 64];
+    __shared__ float plds[PAIR_LDS<LPP, SumDot::NT>];
+    float *const T = pair_part<LPP, SumDot::NT>(plds);
+    if (check_done && (PRESSURE ? D.ctl->done : D.ctl->done_v)) return;
+    const unsigned t = blk * blockDim.x + threadIdx.x;
+    const unsigned i = t / LPP, hl = t % LPP;
+    const bool act = jacobi_takes<PRESSURE>(D, i);
+    float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), ai = xi;
+    unsigned cnt = 0;
+    float s = 0.f;
+    if (act) {
+        xi = D.x[i];
+        ai = D.ap[i];
+        cnt = D.cf[i];
+        aij_sums<LPP>(D, i, hl, cnt, T, xi, ai, &s);
+    }
+    double err, over;
+    jacobi_particle<PRESSURE, LPP>(
+        D, i, hl, act, cnt, xi, ai, s, T, [&] { return jacobi_own<PRESSURE>(D, i); }, err, over);
     const double bs = block_sum(err, lds);
     const double bo = block_sum(over, lds);
     if (threadIdx.x == 0) {
+        D.partial[2 * part] = bs;
+        D.partial[2 * part + 1] = bo;
+    }
+}
+
+// The same for a tile of one model's particles (TILE LPP threads). The error
+// partials are those of the blocks of k_jacobi, in the same places.
+template <bool PRESSURE, int LPP>
+__global__ __launch_bounds__(TILE *LPP) void k_jacobi_tile(Dev D, int check_done) {
+    __shared__ float4 tx[TILE_CAP];  // x, y, z, a.x
+    __shared__ float2 ta[TILE_CAP];  // a.y, a.z
+    __shared__ double lds[2][TILE * LPP / 64];
+    if (check_done && (PRESSURE ? D.ctl->done : D.ctl->done_v)) return;
+    const unsigned blk = xcd_block(), i = blk * TILE + threadIdx.x / LPP, hl = threadIdx.x % LPP;
+    const unsigned m = D.tcount[blk];
+    const bool act = jacobi_takes<PRESSURE>(D, i);
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 xi = act ? D.x[i] : z4, ai = act ? D.ap[i] : z4;
+    const unsigned cnt = act ? D.cf[i] : 0u;
+    const JacobiOwn own = act && hl == 0 ? jacobi_own<PRESSURE>(D, i) : JacobiOwn{0.f, 0.f, 0.f};
+    float s = 0.f;
+    if (m != 0u) {
+        struct XA {
+            float4 x, a;
+        };
+        const F4Gather X(D.x, D.n), A(D.ap, D.n);
+        TileWords<LPP> words(D, i, hl);
+        tile_stage<TILE * LPP>(
+            D, blk, m, [&](unsigned j) { return XA{X.xyz(j), A.xyz(j)}; },
+            [&](unsigned k, const XA &v) {
+                tx[k] = make_float4(v.x.x, v.x.y, v.x.z, v.a.x);
+                ta[k] = make_float2(v.a.y, v.a.z);
+            });
+        __syncthreads();
+        words.pairs(D, hl, cnt, [&](auto... k) {
+            constexpr unsigned N = sizeof...(k);
+            const float4 xj[N] = {tx[k]...};
+            const float2 aj[N] = {ta[k]...};
+            float3 r[N];
+            float g[N];
+            kernel_Gs<N>(xi, xj, D.K, r, g);
+#pragma unroll
+            for (unsigned q = 0; q < N; q++) {
+                const float u[SumDot::NT] = {
+                    g[q], aij_dot(ai, make_float4(xj[q].w, aj[q].x, aj[q].y, 0.f), r[q])};
+                sum_terms<SumDot>(u, &s);
+            }
+        });
+    } else {
+        aij_sums<LPP>(D, i, hl, cnt, nullptr, xi, ai, &s);
+    }
+    double err, over;
+    jacobi_particle<PRESSURE, LPP>(
+        D, i, hl, act, cnt, xi, ai, s, nullptr, [&] { return own; }, err, over);
+    err = wave_sum(err);
+    over = wave_sum(over);
+    const unsigned wid = threadIdx.x >> 6;
+    if ((threadIdx.x & 63u) == 0u) {
+        lds[0][wid] = err;
+        lds[1][wid] = over;
+    }
+    __syncthreads();
+    const unsigned B = (D.n * LPP + BLOCK - 1) / BLOCK, q = (blk * TILE * LPP + threadIdx.x) / BLOCK;
+    if (threadIdx.x % BLOCK == 0 && q < B) {
+        double bs = 0.0, bo = 0.0;
+        for (int w = 0; w < BLOCK / 64; w++) {
+            bs += lds[0][wid + w];
+            bo += lds[1][wid + w];
+        }
+        const unsigned part = xcd_slot(q, B);
         D.partial[2 * part] = bs;
         D.partial[2 * part + 1] = bo;
     }
@@ -2291,6 +2645,10 @@ Dev DFSPH::dev() const {
     D.pv = pv_.get();
     D.nf = nf_.get();
     D.nf16 = use16_ ? nf16_.get() : nullptr;
+    D.nt16 = tiled_ ? nt16_.get() : nullptr;
+    D.tslot = tiled_ ? tslot_.get() : nullptr;
+    D.tcount = tiled_ ? tcount_.get() : nullptr;
+    D.quads16 = (capF_ + 7) / 8;
     D.cf = cf_.get();
     D.nb = nb_l_.get();
     D.cb = cb_.get();
@@ -2626,7 +2984,25 @@ void DFSPH::build_lists() {
         if (!again) break;
     }
     use16_ = hctl_->ovf16 == 0u;
+    build_tiles();
     have_lists_ = true;
+}
+
+// The lists of the iterations' sweeps (single-model scenes whose lists are
+// packed), from the size where the lanes are timed: there a step's dozen or
+// more iterations save 3 us each and the tiles cost 31 us, at 166k 5 against
+// 35, at 1M 45 against 86. Below it the 16 ordered lanes hide the latency
+// that staging would add.
+void DFSPH::build_tiles() {
+    tiled_ = use16_ && !models_ && method_ == SPH_METHOD_DFSPH && n_ >= SMALL_PARTICLES;
+    if (!tiled_) return;
+    const unsigned nt = ((unsigned)n_ + TILE - 1) / TILE;
+    nt16_.reserve(4 * (size_t)((capF_ + 7) / 8) * stride_);
+    tslot_.reserve((size_t)nt * (TILE_CAP / 2));
+    tcount_.reserve(nt);
+    TimedScope ts(timer, stream, "tile_lists");
+    k_tile_lists<<<nt, TILE, 0, stream>>>(dev(), reinterpret_cast<uint4 *>(nt16_.get()), tslot_.get(), tcount_.get());
+    SPH_HIP(hipGetLastError());
 }
 
 // Lanes per particle of a count too small to time. The two give the same
@@ -2836,6 +3212,25 @@ static void launch_sweep(int lanes, unsigned n, hipStream_t s, const Dev &D, int
 #undef SWEEP
     SPH_HIP(hipGetLastError());
 }
+// The same from tiles where the lists have them.
+template <bool PRESSURE, bool JACOBI>
+static void launch_iteration_sweep(int lanes, unsigned n, hipStream_t s, const Dev &D, int check_done) {
+    const unsigned nb = (n + TILE - 1) / TILE;
+#define SWEEP(L)                                                                  \
+    if (lanes == L) {                                                             \
+        if (JACOBI)                                                               \
+            k_jacobi_tile<PRESSURE, L><<<nb, TILE * L, 0, s>>>(D, check_done);    \
+        else                                                                      \
+            k_accel_tile<PRESSURE, L><<<nb, TILE * L, 0, s>>>(D, check_done);     \
+    }
+    if (D.nt16 && lanes <= 4) {
+        SWEEP(1) SWEEP(2) SWEEP(4)
+        SPH_HIP(hipGetLastError());
+    } else {
+        launch_sweep<PRESSURE, JACOBI>(lanes, n, s, D, check_done);
+    }
+#undef SWEEP
+}
 
 // One Jacobi iteration: accelerations, then the update (each sweep with its
 // own lanes per particle).
@@ -2862,11 +3257,11 @@ void DFSPH::iteration_any(bool force) {
     const Dev D = dev();
     {
         TimedScope ts(timer, stream, PRESSURE ? "pressure_accel" : "pressure_accel_v");
-        launch_sweep<PRESSURE, false>(lppA_, (unsigned)n_, stream, D, force ? 0 : 1);
+        launch_iteration_sweep<PRESSURE, false>(lppA_, (unsigned)n_, stream, D, force ? 0 : 1);
     }
     {
         TimedScope ts(timer, stream, PRESSURE ? "jacobi" : "jacobi_v");
-        launch_sweep<PRESSURE, true>(lpp_, (unsigned)n_, stream, D, force ? 0 : 1);
+        launch_iteration_sweep<PRESSURE, true>(lpp_, (unsigned)n_, stream, D, force ? 0 : 1);
     }
     REDUCE("jacobi_reduce", k_jacobi_reduce<PRESSURE>, D, nblocks((size_t)n_ * lpp_), force ? 0 : 1);
 }

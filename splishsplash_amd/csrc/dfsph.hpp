@@ -51,6 +51,16 @@ struct Dev {
     // the low and high halves of nf16[w * stride + i]. The solver sweeps read
     // these -- half the index bytes and index loads of nf.
     const unsigned *nf16;
+    // Tiled lists (null below SMALL_PARTICLES and where nf16 is): the union
+    // of the neighbours of particles b TILE .. b TILE + TILE - 1, tcount[b]
+    // slots (0: more than TILE_CAP, or too far apart), as int16 differences
+    // slot - b TILE, two per word, at tslot[b TILE_CAP / 2]; and the lists
+    // of those particles as 16-bit places in the union, the words of nf16 by
+    // quads: words 4g, 4g + 2, 4g + 1, 4g + 3 of particle i at
+    // nt16[4 (g stride + i)], g < quads16. One, two or four lanes of the
+    // particle then each load their share of a quad at once.
+    const unsigned *nt16, *tslot, *tcount;
+    unsigned quads16;
     const float4 *bx;  // Akinci particles (x, y, z, volume), cell-sorted
     int bmode;         // 0 none, 1 Akinci2012, 2 Bender2019, 3 Koschier2017
     unsigned nvm;      // map slots: vmb[o * stride + i], entries with
@@ -115,6 +125,12 @@ struct EmitterDesc {
     double next = 0;       // m_nextEmitTime
     unsigned counter = 0;  // m_emitCounter
 };
+
+// Particles per tile of the tiled lists, and the slots a tile may gather (see
+// k_tile_lists): a tile along a row of cells of fluid at rest has 1,300 to
+// 1,500, at most 1,930 in a collapsing column. 24 bytes a slot let three
+// blocks of k_jacobi_tile share a CU, 16 five of k_accel_tile.
+constexpr unsigned TILE = 256, TILE_CAP = 1856;
 
 // Below this many particles the lanes per particle follow a rule instead of
 // timings (see DFSPH::tune_lanes).
@@ -294,6 +310,9 @@ private:
     DBuf<unsigned> id_, id2_, nf_, cf_, nb_l_, cb_, bperm_, bstart_;
     DBuf<unsigned> nf16_;    // packed fluid lists (see Dev::nf16)
     bool use16_ = false;     // nf16_ holds the current lists
+    DBuf<unsigned> nt16_, tslot_, tcount_;  // tiled fluid lists (see Dev::nt16)
+    bool tiled_ = false;     // they hold the current lists
+    void build_tiles();
     void ensure_pair_grad();
     DBuf<float4> minv_, cgx_, cgr_, cgp_, cgz_, cgt_;
     DBuf<double> partial_;

@@ -28,6 +28,8 @@ struct KernelConst {
     double invStep_d;   // 1 / (h / 9999) in double, as the reference computes it
     double invStep2_d;  // invStep_d^2
     double h_d;
+    float band;         // half-width of the FP64 band of table_step, per step
+    float G0;           // the gradient entry of step 0: 0.5 (G[0] + G[1]) with G[0] = 0
 };
 
 KernelConst make_kernel_const(double h);
@@ -39,22 +41,29 @@ constexpr unsigned KRES = 10000u;
 // across q = 1/2 and smooth on each side, so the two differ by
 // f'' s^2 / 8, about 1e-8 of the value for s = h / 9999. G[0] = 0 (the
 // reference's special case at r = 0) is kept exactly.
-__device__ __forceinline__ float table_W_avg(unsigned p, const KernelConst &K) {
-    const float q = fmaf((float)p, K.stepq, 0.5f * K.stepq);
-    const float q2 = q * q, f = 1.0f - q;
+//
+// Steps are floats (exact integers). A step past the table (9999 and up)
+// stands for a pair outside the support: 1 - q is clamped to zero, which the
+// subtraction does by itself, and both outer pieces vanish.
+__device__ __forceinline__ float table_f(float q) { return __builtin_amdgcn_fmed3f(1.0f - q, 0.0f, 1.0f); }
+__device__ __forceinline__ float table_W_avg(float p, const KernelConst &K) {
+    const float q = fmaf(p, K.stepq, 0.5f * K.stepq);
+    const float q2 = q * q, f = table_f(q);
     const float inner = K.k * fmaf(6.0f * q2, q - 1.0f, 1.0f);  // 6 q^3 - 6 q^2 + 1
     const float outer = K.k * (2.0f * f * f * f);
     return (q <= 0.5f) ? inner : outer;
 }
 // Both pieces are evaluated and one is selected: the lanes of a wave take
 // both sides of q = 1/2, so a branch would run both anyway.
-__device__ __forceinline__ float table_G_avg(unsigned p, const KernelConst &K) {
-    const float q = (p == 0u) ? K.stepq : fmaf((float)p, K.stepq, 0.5f * K.stepq);
-    const float f = 1.0f - q;
+__device__ __forceinline__ float table_G_past0(float p, const KernelConst &K) {
+    const float q = fmaf(p, K.stepq, 0.5f * K.stepq);
+    const float f = table_f(q);
     const float inner = K.lh2 * fmaf(3.0f, q, -2.0f);
     const float outer = -K.lh2 * f * f * __builtin_amdgcn_rcpf(q);
-    const float g = (q <= 0.5f) ? inner : outer;
-    return (p == 0u) ? 0.5f * g : g;
+    return (q <= 0.5f) ? inner : outer;
+}
+__device__ __forceinline__ float table_G_avg(float p, const KernelConst &K) {
+    return p == 0.0f ? K.G0 : table_G_past0(p, K);
 }
 
 __device__ __forceinline__ float sqn(float x, float y, float z) { return (x * x + y * y) + z * z; }
@@ -63,60 +72,79 @@ __device__ __forceinline__ float sqn(float x, float y, float z) { return (x * x 
 // FP32 expression of the reference's float build).
 __device__ __forceinline__ float sqn_fma(float x, float y, float z) { return fmaf(z, z, fmaf(y, y, x * x)); }
 
-// Table position for the pair (xi, xj) with FP32 squared distance d2. The
-// FP32 value t = |r| / s is within 3.9e-7 t of the FP64 one (coordinate
-// differences, squares and sums: at most 3e-7 on d2, with or without fused
-// multiply-adds, halved by the square root;
-// 1-ulp square root; invStep rounding; product). Inside a band of 5e-7 t
-// around an integer m the step is decided in FP64 from the original FP32
+// Table step of the pair (xi, xj) with FP32 squared distance d2. With
+// u = 2^-24 the FP32 value t = |r| / s is within 5.5 u t plus the rounding of
+// the factor 1 / s of the FP64 one: coordinate differences, squares and sums
+// are at most 5 u on d2, with or without fused multiply-adds, halved by the
+// square root; the root itself is good to one ulp (2 u), the product to u.
+// Inside a band K.band t of that width (3.3e-7 to 3.9e-7) around an integer
+// m the step is decided in FP64 from the original FP32
 // coordinates: floor(|r| / s) >= m  <=>  |r|^2 / s^2 >= m^2, which is what an
 // FP64 build computes from the same positions up to its last-bit rounding.
-__device__ __forceinline__ unsigned table_pos(const float4 &xi, const float4 &xj, float d2, const KernelConst &K) {
+// A wave takes that path for about every third pair (a lane in 150), 12 % of
+// k_jacobi's time.
+// The band around the last entry also decides the support: d2 <= h^2 differs
+// from t <= 9999 by less than the band, so only there the two are compared
+// (inside: at most step 9998; outside: 9999), and everywhere else floor(t)
+// says it. Against a test and a select per pair on top of an integer step
+// with its clamp and conversions: 12 % fewer vector instructions in k_accel
+// (1.71e7 for 1.94e7 a launch at 1M particles), which the gathering sweeps
+// hardly notice (1-2 %) and the tiled ones, bound by them, do.
+__device__ __forceinline__ float table_step(const float4 &xi, const float4 &xj, float d2, const KernelConst &K) {
     const float t = __builtin_amdgcn_sqrtf(d2) * K.invStep_f;
-    unsigned pos = (unsigned)t;
+    float p = floorf(t);
     const float m = rintf(t);
-    if (fabsf(t - m) < fmaf(5.0e-7f, t, 2.0e-6f)) {
+    if (fabsf(t - m) < fmaf(K.band, t, 2.0e-6f)) {
         const double dx = (double)xi.x - (double)xj.x;
         const double dy = (double)xi.y - (double)xj.y;
         const double dz = (double)xi.z - (double)xj.z;
         const double d2d = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
         const double md = (double)m;
-        const unsigned mi = (unsigned)m;
-        pos = (__dmul_rn(d2d, K.invStep2_d) >= md * md) ? mi : mi - 1u;
+        p = (__dmul_rn(d2d, K.invStep2_d) >= md * md) ? m : m - 1.0f;
+        p = (d2 <= K.h2) ? fminf(p, (float)(KRES - 2u)) : (float)(KRES - 1u);
     }
-    return pos < KRES - 2u ? pos : KRES - 2u;
+    return p;
 }
-
-// The kernels below evaluate the table at every pair and select zero outside
-// the support (r^2 > h^2) afterwards: the pairs of a neighbour list are
-// inside, so a branch would only add exec-mask work per pair.
 
 // W(xi - xj); zero outside the support.
 __device__ __forceinline__ float kernel_W(const float4 &xi, const float4 &xj, const KernelConst &K) {
     const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-    const float d2 = sqn_fma(dx, dy, dz);
-    const float w = table_W_avg(table_pos(xi, xj, d2, K), K);
-    return (d2 <= K.h2) ? w : 0.0f;
+    return table_W_avg(table_step(xi, xj, sqn_fma(dx, dy, dz), K), K);
 }
 
 // Scalar g with gradW(xi - xj) = g (xi - xj); zero outside the support.
 // Also returns r = xi - xj.
 __device__ __forceinline__ float kernel_G(const float4 &xi, const float4 &xj, const KernelConst &K, float3 &r) {
     r = make_float3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z);
-    const float d2 = sqn_fma(r.x, r.y, r.z);
-    const float g = table_G_avg(table_pos(xi, xj, d2, K), K);
-    return (d2 <= K.h2) ? g : 0.0f;
+    return table_G_avg(table_step(xi, xj, sqn_fma(r.x, r.y, r.z), K), K);
+}
+
+// kernel_G of N neighbours; whether any pair is within the first step is
+// asked once for all.
+template <unsigned N>
+__device__ __forceinline__ void kernel_Gs(const float4 &xi, const float4 *xj, const KernelConst &K, float3 *r, float *g) {
+    float p[N], p0 = (float)KRES;
+#pragma unroll
+    for (unsigned q = 0; q < N; q++) {
+        r[q] = make_float3(xi.x - xj[q].x, xi.y - xj[q].y, xi.z - xj[q].z);
+        p[q] = table_step(xi, xj[q], sqn_fma(r[q].x, r[q].y, r[q].z), K);
+        g[q] = table_G_past0(p[q], K);
+        p0 = fminf(p0, p[q]);
+    }
+    if (__builtin_expect(p0 == 0.0f, 0)) {
+#pragma unroll
+        for (unsigned q = 0; q < N; q++)
+            if (p[q] == 0.0f) g[q] = K.G0;
+    }
 }
 
 // Both W and the gradient scalar for one pair.
 __device__ __forceinline__ void kernel_WG(const float4 &xi, const float4 &xj, const KernelConst &K, float3 &r, float &w,
                                           float &g) {
     r = make_float3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z);
-    const float d2 = sqn_fma(r.x, r.y, r.z);
-    const unsigned p = table_pos(xi, xj, d2, K);
-    const bool in = d2 <= K.h2;
-    w = in ? table_W_avg(p, K) : 0.0f;
-    g = in ? table_G_avg(p, K) : 0.0f;
+    const float p = table_step(xi, xj, sqn_fma(r.x, r.y, r.z), K);
+    w = table_W_avg(p, K);
+    g = table_G_avg(p, K);
 }
 
 __device__ __forceinline__ float dot3(const float3 &a, const float3 &b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }

@@ -45,6 +45,7 @@ KernelConst make_kernel_const(double h) {
     const double stepSize = h / (double)(KRES - 1);
     K.invStep_d = 1.0 / stepSize;
     K.invStep_f = (float)K.invStep_d;
+    K.band = (float)(1.01 * (5.5 * 0x1p-24 + std::fabs((double)K.invStep_f / K.invStep_d - 1.0)));
     K.invStep2_d = K.invStep_d * K.invStep_d;
     K.k = (float)(8.0 / (pi * h3));
     K.l = (float)(48.0 / (pi * h3));
@@ -53,6 +54,7 @@ KernelConst make_kernel_const(double h) {
     K.lh2 = (float)(48.0 / (pi * h3) / (h * h));
     K.stepq = (float)(1.0 / (double)(KRES - 1));
     K.h_d = h;
+    K.G0 = 0.5f * (K.lh2 * std::fmaf(3.0f, K.stepq, -2.0f));
     return K;
 }
 

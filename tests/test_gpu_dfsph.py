@@ -182,6 +182,54 @@ def test_shared_pairs_sum_as_one_lane(side, kw):
         np.testing.assert_array_equal(sims[0].get(f), sims[1].get(f), err_msg=f)
 
 
+@pytest.mark.parametrize("lanes", [1, 2, 4])
+def test_tiled_sweeps_match_gathered_ones(lanes):
+    # From 65,536 particles on the iterations read neighbours from tiles in
+    # LDS. The same scene with 300 more points in one spot far away keeps no
+    # packed lists, hence no tiles, and gathers. 70,411 particles leave the
+    # last tile ragged, particles strewn alone have no neighbours, and tiles
+    # across thin dense sheets outgrow their share of LDS. With one lane per
+    # particle both take the same sums, bit for bit; with more the gathered
+    # lists are split differently: two orders of at most 128 terms, each
+    # within 127 2^-24 of the terms' absolute sum, which stays below 32 times
+    # the largest result.
+    sc = scenes.dam_break_small(per_side=(44, 40, 38))
+    sheet = scenes.lattice_block((1, 30, 30), 0.02, (2.4, 0.1, 0.1), jitter=0.0005, seed=4)
+    dense = np.concatenate([sheet + np.float32([0.21 * k, 0, 0]) for k in range(7)])
+    alone = scenes.f32([[3.9, 0.1 + 0.15 * k, 1.9] for k in range(11)])
+    x = np.concatenate([sc["x"][:70400 - len(dense)], dense, alone])
+    n = len(x)
+    assert n == 70411
+    spot = np.float32([3.2, 2.6, 1.2]) + np.random.default_rng(8).uniform(-0.01, 0.01, (300, 3)).astype(np.float32)
+    v, p, pv = perturbed_state(x, seed=11)
+    out = []
+    for extra in (np.zeros((0, 3), np.float32), spot):
+        g = capi.TimeStepDFSPH(sc["params"])
+        g.set_fluid(scenes.f32(np.concatenate([x, extra])), scenes.f32(np.concatenate([v, 0 * extra])))
+        g.add_boundary_particles(sc["boundary_x"])
+        g.set_lanes_per_particle(lanes)
+        g.enable_timing()
+        g.init()
+        g.stage("neighborhood_search")
+        assert ("tile_lists" in g.kernel_stats()) == (len(extra) == 0)
+        pad = lambda a: scenes.f32(np.concatenate([a, np.zeros(len(extra), np.float32)]))
+        g.set("p / rho^2", pad(p))
+        g.set("p_v / rho^2", pad(pv))
+        got = {}
+        for stage in ("densities", "dfsph_factor", "divergence_setup", "divergence_iter", "pressure_setup", "pressure_iter",
+                      "pressure_iter"):
+            g.stage(stage)
+            for f in ("pressure acceleration", "p / rho^2", "p_v / rho^2"):
+                got[stage, f] = g.get(f)[:n]
+        out.append(got)
+    for k, a in out[0].items():
+        b = out[1][k]
+        if lanes == 1:
+            np.testing.assert_array_equal(a, b, err_msg=str(k))
+        else:
+            np.testing.assert_allclose(a, b, rtol=0, atol=2 * 127 * 2.0**-24 * 32 * np.abs(b).max(), err_msg=str(k))
+
+
 def vm_scene(n=16, corner=0.06):
     x = scenes.lattice_block((n, n, n), 0.05, (corner, corner, corner), jitter=0.002, seed=5)
     # three particles inside the wall (projected back by the volume-map stage)

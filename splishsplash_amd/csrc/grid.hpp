@@ -79,7 +79,6 @@ void cell_sort_raw(hipStream_t s, const float4 *x, unsigned n, const GridDesc &g
 
 // Gathers dst[k] = src[perm[k]] for k < n.
 void permute_f4(hipStream_t s, const unsigned *perm, unsigned n, const float4 *src, float4 *dst);
-void permute_f1(hipStream_t s, const unsigned *perm, unsigned n, const float *src, float *dst);
 void permute_u1(hipStream_t s, const unsigned *perm, unsigned n, const unsigned *src, unsigned *dst);
 void fill_u32(hipStream_t s, unsigned *p, size_t n, unsigned v);
 

@@ -250,3 +250,21 @@ def test_drop_in_lists_of_two_sets_keep_their_order(n):
     off_e, idx_e = expected_csr(x, r, y)
     np.testing.assert_array_equal(off, off_e)
     np.testing.assert_array_equal(idx, idx_e)
+
+
+@pytest.mark.parametrize("n", [2, 4094, 4096, 4098, 1024 * 4096, 1024 * 4096 + 2])
+def test_list_offsets_at_the_limits_of_the_scans(n):
+    # Pairs of points that see only each other: the offsets are a scan of n
+    # ones, by one block up to 4,096 values, by two launches up to 4,096
+    # tiles of 1,024, by three beyond.
+    k = np.arange(n // 2)
+    a = 0.1 * np.stack([k % 128, k // 128 % 128, k // 16384], 1)
+    x = np.empty((n, 3), np.float32)
+    x[0::2] = a
+    x[1::2] = a + 0.01
+    ns = capi.NeighborhoodSearch(0.05)
+    ns.add_point_set(x)
+    ns.find_neighbors()
+    off, idx = ns.neighbors_csr(0, 0)
+    np.testing.assert_array_equal(off, np.arange(n + 1))
+    np.testing.assert_array_equal(idx, np.arange(n) ^ 1)

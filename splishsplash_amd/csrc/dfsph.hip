@@ -2674,9 +2674,10 @@ Dev DFSPH::dev() const {
     D.pv = pv_.get();
     D.nf = nf_.get();
     D.nf16 = use16_ ? nf16_.get() : nullptr;
-    D.nt16 = tiled_ ? nt16_.get() : nullptr;
-    D.tslot = tiled_ ? tslot_.get() : nullptr;
-    D.tcount = tiled_ ? tcount_.get() : nullptr;
+    const bool tiled = tiled_ && lists_n_ == n_;
+    D.nt16 = tiled ? nt16_.get() : nullptr;
+    D.tslot = tiled ? tslot_.get() : nullptr;
+    D.tcount = tiled ? tcount_.get() : nullptr;
     D.quads16 = (capF_ + 7) / 8;
     D.cf = cf_.get();
     D.nb = nb_l_.get();
@@ -3013,7 +3014,8 @@ void DFSPH::build_lists() {
         k_reset<<<1, 1, 0, stream>>>(ctl_.get(), 2);
     }
     use16_ = hctl_->ovf16 == 0u;
-    build_tiles();
+    tiled_ = tiles_known_ = false;
+    lists_n_ = n_;
     have_lists_ = true;
 }
 
@@ -3022,8 +3024,12 @@ void DFSPH::build_lists() {
 // more iterations save 3 us each and the tiles cost 31 us, at 166k 5 against
 // 35, at 1M 45 against 86. Below it the 16 ordered lanes hide the latency
 // that staging would add.
+// They are built when the first iteration asks for them: a search, a density
+// or a batched solve has no use for them.
 void DFSPH::build_tiles() {
-    tiled_ = use16_ && !models_ && method_ == SPH_METHOD_DFSPH && n_ >= SMALL_PARTICLES;
+    if (tiles_known_) return;
+    tiles_known_ = true;
+    tiled_ = have_lists_ && lists_n_ == n_ && use16_ && !models_ && method_ == SPH_METHOD_DFSPH && n_ >= SMALL_PARTICLES;
     if (!tiled_) return;
     const unsigned nt = ((unsigned)n_ + TILE - 1) / TILE;
     nt16_.reserve(4 * (size_t)((capF_ + 7) / 8) * stride_);
@@ -3279,6 +3285,7 @@ void DFSPH::iteration_any(bool force) {
         }
         return;
     }
+    build_tiles();
     const Dev D = dev();
     {
         TimedScope ts(timer, stream, PRESSURE ? "pressure_accel" : "pressure_accel_v");

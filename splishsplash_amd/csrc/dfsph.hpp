@@ -312,6 +312,8 @@ private:
     bool use16_ = false;     // nf16_ holds the current lists
     DBuf<unsigned> nt16_, tslot_, tcount_;  // tiled fluid lists (see Dev::nt16)
     bool tiled_ = false;     // they hold the current lists
+    size_t lists_n_ = 0;     // particles the current lists were built for
+    bool tiles_known_ = false;  // whether they do has been settled for these lists
     void build_tiles();
     void ensure_pair_grad();
     DBuf<float4> minv_, cgx_, cgr_, cgp_, cgz_, cgt_;

@@ -434,7 +434,7 @@ int sph_dfsph_get_body_reference(sph_dfsph_t s, unsigned obj, double position[3]
  * steps. In batch modes 1 and 2 the two solves of a step run
  * for all scenes at once: each Jacobi iteration is one acceleration sweep
  * and one update over every scene's particles plus one reduction block per
- * scene, scenes grouped by their tuned lanes per particle, converged scenes
+ * scene, scenes grouped by their lanes per particle, converged scenes
  * returning at entry; mode 2 replays the iterations between two convergence
  * checks from captured HIP graphs. The rest of each step runs per scene on
  * its own stream over `threads` host threads (0: up to 16). This needs
@@ -443,7 +443,7 @@ int sph_dfsph_get_body_reference(sph_dfsph_t s, unsigned obj, double position[3]
  * solver; otherwise, and in mode 0, the handles are shared out over the
  * host threads by particle count and each thread interleaves its scenes
  * step by step. Each scene's results are those of sph_dfsph_step on it
- * alone with the same lanes per particle. When some handle has yet to time
+ * alone with the same lanes per particle. When some handle has yet to pick
  * its lanes per particle (its first step after creation or after lanes 0 was
  * set), every handle first takes one step here, one handle at a time, and
  * the mode runs the remaining n_steps - 1. A handle may appear once; the
@@ -490,11 +490,14 @@ int sph_dfsph_enable_timing(sph_dfsph_t s, int enable);
  * those kernels only. */
 int sph_dfsph_time_only(sph_dfsph_t s, const char *names);
 /* Lanes per particle of the sweeps: 1, 2 or 4 for all of them, or 0
- * (default) to let the first solve time the choices on the live state and
- * keep the fastest, separately for the acceleration sweeps and the Jacobi
- * update (whose choice the other sweeps follow). Small counts are not timed:
- * up to 40,960 particles (of all scenes stepped together) 16 lanes share a
- * particle's pairs, and its sums are those of one lane. */
+ * (default) to leave them to a rule on the particle count and the lists, for
+ * the acceleration sweeps and for the Jacobi update (which the other sweeps
+ * follow). They fix the order of the FP32 neighbour sums. From 65,536
+ * particles on the rule is applied at the first sweep and its choice kept
+ * until the caller adds particles (sph_dfsph_emit_particles, a longer state
+ * file) or sets lanes again; below, one lane's sums are taken, up to 40,960
+ * particles (of all scenes stepped together) by 16 lanes that share a
+ * particle's pairs. */
 int sph_dfsph_set_lanes_per_particle(sph_dfsph_t s, int lanes);
 int sph_dfsph_kernel_stats(sph_dfsph_t s, int k, const char **name,
                            long long *launches, double *total_ms,

@@ -777,7 +777,7 @@ class TimeStepDFSPH:
         _chk(lib().sph_dfsph_enable_timing(self.h, int(on)))
 
     def set_lanes_per_particle(self, lanes):
-        """1, 2 or 4 lanes per particle in the solver sweeps; 0 = autotune."""
+        """1, 2 or 4 lanes per particle in the solver sweeps; 0: by rule."""
         _chk(lib().sph_dfsph_set_lanes_per_particle(self.h, int(lanes)))
 
     def time_only(self, names):

@@ -11,8 +11,8 @@
 // reduction block per scene), reading the scenes' states from a device
 // table, and a scene whose solve has converged returns at entry. The
 // iterations between two convergence checks are captured once as a HIP
-// graph and replayed. Scenes are grouped by their lanes per particle (each
-// scene's autotuned choice), one batch per group.
+// graph and replayed. Scenes are grouped by their lanes per particle, one
+// batch per group.
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
@@ -248,9 +248,9 @@ struct BatchRunner {
         }
     }
 
-    // Groups and block maps (after the tuner has picked each scene's lanes).
+    // Groups and block maps (once each scene's lanes are known).
     void setup(const std::vector<DFSPH *> &all) {
-        // group by the lanes each scene's tuner picked
+        // group by the scenes' lanes
         std::map<std::pair<int, int>, std::vector<DFSPH *>> by;
         for (DFSPH *s : all) by[{s->lanes_accel(), s->lanes_jacobi()}].push_back(s);
         bool same = by.size() == groups.size();
@@ -360,11 +360,10 @@ struct BatchRunner {
         std::vector<char> div(all.size(), 0);
         std::vector<int> its(all.size(), 0);
         parallel_scenes(all.size(), [&](size_t k) {
-            all[k]->ensure_tuned();
             div[k] = all[k]->step_begin() ? 1 : 0;
             SPH_HIP(hipEventRecord(ev[k], all[k]->stream));
         });
-        setup(all);  // the tuner may have changed a scene's lanes
+        setup(all);  // a search may have changed a scene's lanes
         bool anydiv = false;
         for (char d : div) anydiv = anydiv || d;
         if (anydiv) {

@@ -1318,14 +1318,6 @@ __global__ void k_set_time(Ctl *C, double t, double h) {
     C->h = h;
 }
 
-// Tuning input: positions with a unit stiffness in w.
-__global__ __launch_bounds__(BLOCK) void k_unit_w(const float4 *__restrict__ x, float4 *__restrict__ y, unsigned n) {
-    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 a = x[i];
-    y[i] = make_float4(a.x, a.y, a.z, 1.0f);
-}
-
 // divergenceSolve / pressureSolve finalisation (TimeStepDFSPH.cpp:345-383,
 // 500-540): v += h a_p; the divergence solve also restores alpha *= h.
 template <bool PRESSURE, int LPP>
@@ -3014,13 +3006,14 @@ void DFSPH::build_lists() {
         k_reset<<<1, 1, 0, stream>>>(ctl_.get(), 2);
     }
     use16_ = hctl_->ovf16 == 0u;
+    lists_max_ = hctl_->maxcnt_f;
     tiled_ = tiles_known_ = false;
     lists_n_ = n_;
     have_lists_ = true;
 }
 
 // The lists of the iterations' sweeps (single-model scenes whose lists are
-// packed), from the size where the lanes are timed: there a step's dozen or
+// packed), from SMALL_PARTICLES on: there a step's dozen or
 // more iterations save 3 us each and the tiles cost 31 us, at 166k 5 against
 // 35, at 1M 45 against 86. Below it the 16 ordered lanes hide the latency
 // that staging would add.
@@ -3040,7 +3033,7 @@ void DFSPH::build_tiles() {
     SPH_HIP(hipGetLastError());
 }
 
-// Lanes per particle of a count too small to time. The two give the same
+// Lanes per particle of a small count. The two give the same
 // sums bit for bit, so the rule only weighs time: shared pairs hide the
 // memory latency of a nearly idle GPU and cost three times the instructions.
 // Whole steps (us), one lane / shared, Akinci walls and plain start: 2,197
@@ -3053,7 +3046,7 @@ static int small_lanes(size_t n) { return n <= ORDERED_MAX ? ORDERED_LANES : 1; 
 
 void DFSPH::neighborhood_search() {
     if (!initialized_) init();
-    if (!lpp_fixed_ && !timed_) lpp_ = lppA_ = small_lanes(std::max(n_, company_));
+    if (!lpp_fixed_ && !picked_large_) lpp_ = lppA_ = small_lanes(std::max(n_, company_));
     const unsigned n = (unsigned)n_;
     fsort_.sort(stream, x_.get(), n, grid_, timer);
     {
@@ -3217,7 +3210,7 @@ void DFSPH::sweep_init_l(bool dens, bool fact, bool div) {
 }
 
 void DFSPH::sweep_init(bool dens, bool fact, bool div) {
-    if (!tuned_ && have_lists_) tune_lanes();
+    if (!picked_ && have_lists_) pick_lanes();
     if (lpp_ == ORDERED_LANES)
         sweep_init_l<ORDERED_LANES>(dens, fact, div);
     else if (lpp_ == 4)
@@ -3348,61 +3341,34 @@ void DFSPH::div_iteration(bool force) { iteration_any<false>(force); }
 
 void DFSPH::pressure_iteration(bool force) { iteration_any<true>(force); }
 
-// Picks the lanes per particle of the acceleration sweeps and of the Jacobi
-// update (used for the other sweeps too) by timing each sweep for 1, 2 and 4
-// lanes on the current neighbour lists, best of three launches each. The
-// sweeps read a uniform stiffness (every pair active) from scratch copies of
-// the positions and stiffness and write to those copies, a scratch
-// acceleration array and the reduction partials, none of which holds state
-// between solves.
-void DFSPH::tune_lanes() {
-    tuned_ = true;
+// The lanes per particle of a large scene (from SMALL_PARTICLES on), by a rule
+// on its count and lists at the first sweep, kept until the caller adds
+// particles or sets lanes. The lanes fix the order of every FP32 neighbour
+// sum, and velocities differ by about a per cent after some tens of steps in
+// another order: a choice by timings made results depend on the noise of
+// those timings (85k particles: four choices in twelve fresh handles).
+// The lines are where the gathering sweeps cross (us at 1 / 2 / 4 lanes,
+// collapsing dam in a box, k_accel with every pair active and k_jacobi):
+//  - Jacobi and the other sweeps: 4 lanes below 84k particles, 2 above
+//    (k_jacobi 69k 16.6 / 14.2 / 13.9, 85k 16.7 / 14.1 / 14.2, 111k 17.5 /
+//    17.0 / 17.5, 1M 78.6 / 66.1 / 83.0);
+//  - accelerations: 4 below 112k (111k 11.9 / 10.7 / 10.4), 2 below 236k
+//    (176k 14.6 / 14.4 / 14.3), above it 1, the fastest with every pair
+//    active (in a flow, where many pairs carry no pressure, 2 lanes gain up
+//    to 10 %: 1M 42.0 / 37.8 / 43.4), but 2 from 32-bit lists (4M 274 / 241 /
+//    270);
+//  - long lists (88 or more: dense clouds; fluid at rest has 53 at most) take
+//    4 for both (70k points, K = 100: k_jacobi 46.8 / 29.8 / 25.0, 500k 160 /
+//    131 / 119).
+// The tiled sweeps of the iterations differ less between 1 and 2 lanes (1M:
+// k_accel_tile 27.3 / 25.4, k_jacobi_tile 54.4 / 49.7) and keep this order.
+void DFSPH::pick_lanes() {
+    picked_ = true;
     if (n_ < SMALL_PARTICLES || lpp_fixed_) return;
-    timed_ = true;
-    Dev D = dev();
-    fill_u32(stream, reinterpret_cast<unsigned *>(p2_.get()), n_, 0x3f800000u);  // 1.0f
-    k_unit_w<<<nblocks(n_), BLOCK, 0, stream>>>(x_.get(), x2_.get(), (unsigned)n_);
-    SPH_HIP(hipGetLastError());
-    D.p = p2_.get();
-    D.x = x2_.get();
-    // a scratch acceleration array: with several fluid models ap_ carries
-    // the other models' accelerations into the next solve
-    DBuf<float4> scratch_ap;
-    scratch_ap.reserve(stride_);
-    D.ap = scratch_ap.get();
-    hipEvent_t a, b;
-    SPH_HIP(hipEventCreate(&a));
-    SPH_HIP(hipEventCreate(&b));
-    int pick[2] = {1, 1};
-    for (int sweep = 0; sweep < 2; sweep++) {
-        float best = 1e30f;
-        for (int L : {1, 2, 4}) {
-            float tmin = 1e30f;
-            for (int rep = 0; rep < 3; rep++) {
-                SPH_HIP(hipEventRecord(a, stream));
-                if (sweep == 0)
-                    launch_sweep<true, false>(L, (unsigned)n_, stream, D, 0);
-                else
-                    launch_sweep<true, true>(L, (unsigned)n_, stream, D, 0);
-                SPH_HIP(hipEventRecord(b, stream));
-                SPH_HIP(hipEventSynchronize(b));
-                float ms = 0.f;
-                SPH_HIP(hipEventElapsedTime(&ms, a, b));
-                tmin = std::min(tmin, ms);
-            }
-            tune_ms_[sweep][L == 1 ? 0 : (L == 2 ? 1 : 2)] = tmin;
-            if (tmin < best) {
-                best = tmin;
-                pick[sweep] = L;
-            }
-        }
-        // the Jacobi sweeps are timed on the accelerations of the chosen lanes
-        if (sweep == 0) launch_sweep<true, false>(pick[0], (unsigned)n_, stream, D, 0);
-    }
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
-    lppA_ = pick[0];
-    lpp_ = pick[1];
+    picked_large_ = true;
+    const bool longl = lists_max_ >= 88u;
+    lpp_ = longl || n_ < 84000 ? 4 : 2;
+    lppA_ = longl || n_ < 112000 ? 4 : (n_ < 236000 || !use16_ ? 2 : 1);
 }
 
 void DFSPH::set_lanes_per_particle(int lpp) {
@@ -3410,8 +3376,8 @@ void DFSPH::set_lanes_per_particle(int lpp) {
     lpp_fixed_ = lpp != 0;
     lpp_ = lpp ? lpp : 1;
     lppA_ = lpp_;
-    tuned_ = lpp_fixed_;
-    timed_ = false;
+    picked_ = lpp_fixed_;
+    picked_large_ = false;
 }
 
 void DFSPH::div_finish(bool scale_pv) {
@@ -3804,7 +3770,7 @@ void DFSPH::stiff_to_w(bool pressure) {
 }
 
 int DFSPH::run_solver(bool pressure, int already, bool copy_w) {
-    if (!tuned_) tune_lanes();
+    if (!picked_) pick_lanes();
     if (copy_w) stiff_to_w(pressure);
     const int maxIt = pressure ? P.max_iterations : P.max_iterations_v;
     int launched = already;

@@ -132,8 +132,9 @@ struct EmitterDesc {
 // blocks of k_jacobi_tile share a CU, 16 five of k_accel_tile.
 constexpr unsigned TILE = 256, TILE_CAP = 1856;
 
-// Below this many particles the lanes per particle follow a rule instead of
-// timings (see DFSPH::tune_lanes).
+// Below this many particles the lanes per particle only weigh time (see
+// small_lanes), from it on they fix the order of the sums (see
+// DFSPH::pick_lanes).
 constexpr size_t SMALL_PARTICLES = 65536;
 
 class DFSPH;
@@ -205,16 +206,13 @@ public:
     void step_after_pressure(int iterations);
     int first_chunk(bool pressure) const;  // iterations launched before the first convergence check
     int solve_result(bool pressure, bool read = true);  // the solver counters (read back first)
-    void ensure_tuned() {
-        if (!tuned_) tune_lanes();
-    }
     // Particles of all scenes stepped together with this one (0: alone).
     void set_company(size_t n) { company_ = n; }
     int lanes_accel() const { return lppA_; }
     int lanes_jacobi() const { return lpp_; }
     Dev device_state() const { return dev(); }
     bool batchable() const;  // the plain DFSPH step with the reference's warm starts
-    bool tuning_pending() const { return !tuned_; }  // the next step times the lanes per particle
+    bool first_step_pending() const { return !picked_; }  // the next step sets up and picks the lanes per particle
     bool any_xsph() const;   // XSPH acts in some fluid model
     unsigned long long serial() const { return serial_; }  // unique per handle in the process
     // Simulation::setSimulationMethod for this handle: SPH_METHOD_DFSPH,
@@ -313,6 +311,7 @@ private:
     DBuf<unsigned> nt16_, tslot_, tcount_;  // tiled fluid lists (see Dev::nt16)
     bool tiled_ = false;     // they hold the current lists
     size_t lists_n_ = 0;     // particles the current lists were built for
+    unsigned lists_max_ = 0;  // the longest of them
     bool tiles_known_ = false;  // whether they do has been settled for these lists
     void build_tiles();
     void ensure_pair_grad();
@@ -392,17 +391,16 @@ private:
     void stiff_to_w(bool pressure);
     template <bool PRESSURE>
     void iteration_any(bool force);
-    void tune_lanes();
+    void pick_lanes();
     int lpp_ = 1;              // lanes per particle of the Jacobi update and the other sweeps
-    int seq_lanes() const { return lpp_ > 4 ? lpp_ : 1; }  // of the sweeps that are not timed (plain sequential sums)
+    int seq_lanes() const { return lpp_ > 4 ? lpp_ : 1; }  // of the sweeps with plain sequential sums at every count
     int lppA_ = 1;             // lanes per particle of the acceleration sweeps (iterations, finish)
     size_t company_ = 0;
-    bool tuned_ = false, timed_ = false, lpp_fixed_ = false;  // timed_: lpp_ and lppA_ come from timings
+    bool picked_ = false, picked_large_ = false, lpp_fixed_ = false;  // picked_large_: at a large count (pick_lanes)
 
 public:
-    float tune_ms_[2][3] = {};  // acceleration / Jacobi sweep time at 1, 2, 4 lanes per particle
     int lanes_per_particle() const { return lpp_; }
-    // 1, 2 or 4 fixes the lanes per particle; 0 lets the first solve pick.
+    // 1, 2 or 4 fixes the lanes per particle; 0 leaves them to the rules.
     void set_lanes_per_particle(int lpp);
 
 private:

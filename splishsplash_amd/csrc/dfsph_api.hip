@@ -285,7 +285,7 @@ void step_threads(sph_dfsph_t *handles, size_t n, int n_steps, size_t T) {
 
 // Mode 3: the first steps of a set of scenes alternate between scene by
 // scene on host threads and batched solves from graphs, one step timed per
-// way after one untimed (set-up, graph capture, lane tuning); the faster way
+// way after one untimed (set-up, graph capture); the faster way
 // runs from then on. A different set of handles is timed again.
 struct AutoChoice {
     std::vector<unsigned long long> ids;
@@ -321,12 +321,13 @@ int sph_dfsph_step_batch(sph_dfsph_t *handles, size_t n, int n_steps, int thread
                 for (size_t k = 0; k < n; k++) h[k]->s->set_company(0);
             }
         } company(handles, n);
-        // A first step that times the sweeps for the lanes per particle runs
-        // here for every handle, one handle at a time, before host threads
-        // or batched solves take over: lane tuning runs with one handle
-        // stepping at a time.
+        // A first step sets a handle up (boundary maps, buffers, list room)
+        // and picks its lanes per particle, by which batched solves group the
+        // scenes: it runs here for every handle, one handle at a time, before
+        // host threads or batched solves take over. (A run whose fresh
+        // handles took first steps concurrently has faulted, cause not found.)
         bool pending = false;
-        for (size_t k = 0; k < n; k++) pending = pending || handles[k]->s->tuning_pending();
+        for (size_t k = 0; k < n; k++) pending = pending || handles[k]->s->first_step_pending();
         if (pending) {
             for (size_t k = 0; k < n; k++) handles[k]->s->step();
             for (size_t k = 0; k < n; k++) handles[k]->s->sync();

@@ -265,7 +265,7 @@ void DFSPH::emit_particles(const float *x, const float *v, size_t k) {
     n_ = n + k;
     cap_emit_ += k;
     have_lists_ = false;
-    tuned_ = lpp_fixed_;
+    picked_ = lpp_fixed_;
 }
 
 // EmitterSystem::step (EmitterSystem.cpp:54-80) at the end of a step, before

@@ -12,7 +12,7 @@ import pytest
 
 from oracle import oracle
 from splishsplash_amd import capi, scenes
-from splishsplash_amd.params import BOUNDARY_BENDER2019, VISCOSITY_STANDARD, VISCOSITY_WEILER2018, default_params
+from splishsplash_amd.params import BOUNDARY_BENDER2019, BOUNDARY_NONE, VISCOSITY_STANDARD, VISCOSITY_WEILER2018, default_params
 
 pytestmark = pytest.mark.gpu
 
@@ -180,6 +180,41 @@ def test_shared_pairs_sum_as_one_lane(side, kw):
         assert sims[0].get("fluid neighbor count").max() > 64
     for f in ("position", "velocity", "density", "factor", "p / rho^2", "p_v / rho^2", "pressure acceleration"):
         np.testing.assert_array_equal(sims[0].get(f), sims[1].get(f), err_msg=f)
+
+
+@pytest.mark.parametrize("dims, n, lanes", [
+    ((42, 40, 40), 65535, (1, 1)), ((42, 40, 40), 65536, (4, 4)), ((44, 44, 44), 83999, (4, 4)),
+    ((44, 44, 44), 84000, (2, 4)), ((49, 49, 49), 111999, (2, 4)), ((49, 49, 49), 112000, (2, 2)),
+    ((62, 62, 62), 235999, (2, 2)), ((62, 62, 62), 236000, (2, 1)), ((240, 100, 10), 240000, (2, 2))])
+def test_lanes_of_large_scenes_follow_their_rule(dims, n, lanes):
+    # The lanes fix the order of the sums, so they come from the count and
+    # the lists alone and every handle with the same particles takes the
+    # same: on both sides of each line, with packed lists and (the wide flat
+    # block, 48,000 slots a layer of cells) with 32-bit ones.
+    x = scenes.lattice_block(dims, 0.05, (0.0, 0.0, 0.0), jitter=0.001, seed=1)[:n]
+    got = []
+    for _ in range(3):
+        g = capi.TimeStepDFSPH(default_params(boundary_handling_method=BOUNDARY_NONE))
+        g.set_fluid(x)
+        g.step(1)
+        c = g.counters()
+        got.append((c["lanes_per_particle"], c["lanes_per_particle_accel"], c["packed_lists"]))
+    assert got == [(*lanes, int(dims[0] < 100))] * 3
+
+
+def test_lanes_of_long_lists_follow_their_rule():
+    # Four lanes from lists of 88 neighbours on, at any count: a block of
+    # 240,000 particles with 1 to 88 more in one spot beside it.
+    block = scenes.lattice_block((63, 63, 63), 0.05, (0.0, 0.0, 0.0), jitter=0.001, seed=1)[:240000]
+    spot = np.float32([1.5, 1.5, -1.0]) + np.random.default_rng(8).uniform(-0.01, 0.01, (89, 3)).astype(np.float32)
+    for k, lanes in ((1, (2, 1)), (88, (2, 1)), (89, (4, 4))):
+        g = capi.TimeStepDFSPH(default_params(boundary_handling_method=BOUNDARY_NONE))
+        g.set_fluid(scenes.f32(np.concatenate([block, spot[:k]])))
+        g.stage("neighborhood_search")
+        g.stage("densities")
+        c = g.counters()
+        assert g.get("fluid neighbor count").max() == max(32, k - 1)
+        assert (c["lanes_per_particle"], c["lanes_per_particle_accel"]) == lanes
 
 
 @pytest.mark.parametrize("lanes", [1, 2, 4])

@@ -197,21 +197,21 @@ __global__ void k_mlp_pack(const float *__restrict__ th, short *__restrict__ pk)
     if (k < MLP_NPARAM) pack_param(k, th[k], pk);
 }
 
-// Gradients of sum_i (y_i - t_i)^2 / n, one partial vector per block. Each
-// tile keeps the activations' derivatives (and h1 in LDS, h2 in registers)
-// from the forward pass, and the waves of a block add their sums in LDS
-// before one of them is written: 128 partials of 18.7 KB for 16,384 rows
-// instead of 512. 16,384 rows: 34.6 us before, 17 us now.
+// A wave's partial sums: the parameters' gradients, then the loss, in rows of
+// whole 128-byte lines.
+constexpr int PART_STRIDE = (MLP_NPARAM + 1 + 31) / 32 * 32;
+
+// Gradients of sum_i (y_i - t_i)^2 / n, one partial row per wave. Each tile
+// keeps the activations' derivatives (and h1 in LDS, h2 in registers) from
+// the forward pass. 16,384 rows: 34.6 us before, 19 us now.
 __global__ __launch_bounds__(64 * MWAVES) void k_mlp_grad(const float *__restrict__ th, const short *__restrict__ pk,
                                                          const float *__restrict__ X, const float *__restrict__ T,
-                                                         unsigned n, float *__restrict__ partial,
-                                                         float *__restrict__ lossp) {
+                                                         unsigned n, float *__restrict__ partial) {
     __shared__ short sm[MWAVES][32 * SP];  // h1
     __shared__ short sd[MWAVES][32 * SP];  // h2, then dz2, then dz1
     __shared__ float xf[MWAVES][32 * MLP_XSTRIDE];
     __shared__ float sy[MWAVES][32];
     __shared__ uint4 W[PACK_GROUPS * 64];
-    __shared__ float G[MWAVES][MLP_NPARAM + 1];
     const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
     for (int k = threadIdx.x; k < PACK_GROUPS * 64; k += 64 * MWAVES) W[k] = reinterpret_cast<const uint4 *>(pk)[k];
     // group c of the packed weights, read where a tile needs it: the
@@ -381,105 +381,91 @@ __global__ __launch_bounds__(64 * MWAVES) void k_mlp_grad(const float *__restric
         }
         wave_sync();
     }
-    // the waves' sums, added in wave order
-    float *const Gw = G[wid];
+    float *const P = partial + (size_t)(blockIdx.x * MWAVES + wid) * PART_STRIDE;
 #pragma unroll
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int e = 0; e < 16; e++) {
             const int m = crow(e, g);
-            if (m < MLP_NIN) Gw[MLP_OFF_W1 + m * 64 + 32 * h + r] = gW1[h][e];
+            if (m < MLP_NIN) P[MLP_OFF_W1 + m * 64 + 32 * h + r] = gW1[h][e];
         }
 #pragma unroll
     for (int mh = 0; mh < 2; mh++)
 #pragma unroll
         for (int nh = 0; nh < 2; nh++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) Gw[MLP_OFF_W2 + (32 * mh + crow(e, g)) * 64 + 32 * nh + r] = gW2[mh][nh][e];
+            for (int e = 0; e < 16; e++) P[MLP_OFF_W2 + (32 * mh + crow(e, g)) * 64 + 32 * nh + r] = gW2[mh][nh][e];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         const float v3 = gW3[h] + __shfl_xor(gW3[h], 32, 64);
         const float v1 = gb1[h] + __shfl_xor(gb1[h], 32, 64);
         const float v2 = gb2[h] + __shfl_xor(gb2[h], 32, 64);
         if (g == 0) {
-            Gw[MLP_OFF_W3 + 32 * h + r] = v3;
-            Gw[MLP_OFF_B1 + 32 * h + r] = v1;
-            Gw[MLP_OFF_B2 + 32 * h + r] = v2;
+            P[MLP_OFF_W3 + 32 * h + r] = v3;
+            P[MLP_OFF_B1 + 32 * h + r] = v1;
+            P[MLP_OFF_B2 + 32 * h + r] = v2;
         }
     }
     const float v3 = gb3 + __shfl_xor(gb3, 32, 64);
     const float l2 = L + __shfl_xor(L, 32, 64);
     if (lane == 0) {
-        Gw[MLP_OFF_B3] = v3;
-        Gw[MLP_NPARAM] = l2;
-    }
-    __syncthreads();
-    float *P = partial + (size_t)blockIdx.x * MLP_NPARAM;
-    for (int k = threadIdx.x; k <= MLP_NPARAM; k += 64 * MWAVES) {
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < MWAVES; w++) v += G[w][k];
-        if (k < MLP_NPARAM)
-            P[k] = v;
-        else
-            lossp[blockIdx.x] = v;
+        P[MLP_OFF_B3] = v3;
+        P[MLP_NPARAM] = l2;
     }
 }
 
-// grad[k] = sum over blocks of partial[b][k], loss = sum(lossp) / n; with
-// ADAM also the parameter update and its packed copy. One wave per 64
-// parameters would walk the partials one after the other (136 us for 512 of
-// them): RSLICES slices of a block take every RSLICES-th partial, their sums
-// are added in slice order. 4.6 us for 128 partials, the update (5 us as a
-// kernel of its own) included.
-constexpr int RSLICES = 16;
+// grad[k] = sum over waves of partial[w][k], one wave's after the other;
+// loss = the same of the last column / n; with ADAM also the parameter update
+// and its packed copy. A lane that loads what it adds takes 136 us for 512
+// rows: here a block stages REDUCE_ROWS rows of 32 columns in LDS, 16 loads
+// of every thread in flight, and 32 lanes add them from there, which is bound
+// by the chain of dependent adds. 7.2 us for 512 rows, the update (5 us as
+// a kernel of its own) included. Sums by block or by slices would be shorter
+// (4.6 us) but add in another order.
+constexpr int REDUCE_COLS = 32, REDUCE_ROWS = 512, REDUCE_THREADS = 1024;
 struct AdamArgs {
     float *th, *m, *v;
     short *pk;
     float b1t, b2t, lr;
 };
 template <bool ADAM>
-__global__ __launch_bounds__(64 * RSLICES) void k_mlp_grad_reduce(const float *__restrict__ partial,
-                                                                 const float *__restrict__ lossp, unsigned nparts,
-                                                                 unsigned n, float *__restrict__ grad,
-                                                                 float *__restrict__ loss, AdamArgs A) {
-    __shared__ float sum[RSLICES][64], ls[64 * RSLICES];
-    const unsigned lane = threadIdx.x & 63u, sl = threadIdx.x >> 6;
-    const unsigned k = blockIdx.x * 64u + lane;
-    float s = 0.f;
-    if (k < (unsigned)MLP_NPARAM) {
-        unsigned b = sl;
-        for (; b + 7 * RSLICES < nparts; b += 8 * RSLICES) {
-            float t[8];
+__global__ __launch_bounds__(REDUCE_THREADS) void k_mlp_grad_reduce(const float *__restrict__ partial, unsigned nparts,
+                                                                   unsigned n, float *__restrict__ grad,
+                                                                   float *__restrict__ loss, AdamArgs A) {
+    constexpr unsigned STEP = REDUCE_THREADS / REDUCE_COLS, PER = REDUCE_ROWS / STEP;
+    __shared__ float T[REDUCE_ROWS][REDUCE_COLS];
+    const unsigned c = threadIdx.x % REDUCE_COLS, r0 = threadIdx.x / REDUCE_COLS;
+    const unsigned k = blockIdx.x * REDUCE_COLS + c;
+    float v[PER], s = 0.f;
+    auto load = [&](unsigned w0) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) t[q] = partial[(size_t)(b + q * RSLICES) * MLP_NPARAM + k];
-#pragma unroll
-            for (int q = 0; q < 8; q++) s += t[q];
+        for (unsigned q = 0; q < PER; q++) {
+            const unsigned w = w0 + q * STEP + r0;
+            v[q] = partial[(size_t)(w < nparts ? w : nparts - 1u) * PART_STRIDE + k];
         }
-        for (; b < nparts; b += RSLICES) s += partial[(size_t)b * MLP_NPARAM + k];
-    }
-    sum[sl][lane] = s;
-    if (blockIdx.x == 0) {
-        float l = 0.f;
-        for (unsigned b = threadIdx.x; b < nparts; b += 64 * RSLICES) l += lossp[b];
-        ls[threadIdx.x] = l;
-    }
-    __syncthreads();
-    if (blockIdx.x == 0 && sl == 1) {
-        float l = 0.f;
+    };
+    load(0);
+    for (unsigned w0 = 0; w0 < nparts; w0 += REDUCE_ROWS) {
+        if (w0) __syncthreads();
 #pragma unroll
-        for (unsigned q = 0; q < RSLICES; q++) l += ls[64 * q + lane];
-        for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
-        if (lane == 0) *loss = l / (float)n;
+        for (unsigned q = 0; q < PER; q++) T[q * STEP + r0][c] = v[q];
+        __syncthreads();
+        if (w0 + REDUCE_ROWS < nparts) load(w0 + REDUCE_ROWS);
+        if (r0 == 0) {
+            const unsigned m = nparts - w0 < (unsigned)REDUCE_ROWS ? nparts - w0 : REDUCE_ROWS;
+#pragma unroll 16
+            for (unsigned w = 0; w < m; w++) s += T[w][c];
+        }
     }
-    if (sl != 0 || k >= (unsigned)MLP_NPARAM) return;
-    float g = 0.f;
-#pragma unroll
-    for (int q = 0; q < RSLICES; q++) g += sum[q][lane];
-    grad[k] = g;
+    if (r0 != 0 || k > (unsigned)MLP_NPARAM) return;
+    if (k == (unsigned)MLP_NPARAM) {
+        *loss = s / (float)n;
+        return;
+    }
+    grad[k] = s;
     if (ADAM) {
-        const float mk = 0.9f * A.m[k] + 0.1f * g;
-        const float vk = 0.999f * A.v[k] + 0.001f * g * g;
+        const float mk = 0.9f * A.m[k] + 0.1f * s;
+        const float vk = 0.999f * A.v[k] + 0.001f * s * s;
         A.m[k] = mk;
         A.v[k] = vk;
         const float t = A.th[k] - A.lr * (mk / (1.0f - A.b1t)) / (sqrtf(vk / (1.0f - A.b2t)) + 1e-8f);
@@ -503,6 +489,8 @@ static unsigned mlp_blocks(unsigned n) {
     return std::max(1u, std::min(1024u, (tiles + MWAVES - 1) / MWAVES));
 }
 
+static unsigned grad_blocks(unsigned n) { return std::min(256u, mlp_blocks(n)); }
+
 void mlp_forward(hipStream_t s, const float *theta, const float *x, unsigned n, float *y) {
     if (!n) return;
     k_mlp_fwd<<<mlp_blocks(n), 64 * MWAVES, 0, s>>>(theta, x, n, y);
@@ -517,25 +505,26 @@ void MLPTrainer::pack(hipStream_t s, const float *theta) {
 
 void MLPTrainer::sums(hipStream_t s, const float *theta, const float *x, const float *t, unsigned n) {
     SPH_REQUIRE(n > 0, SPH_ERR_INVALID, "empty training batch");
-    parts = std::min(256u, mlp_blocks(n));
-    partial.reserve((size_t)parts * MLP_NPARAM);
-    loss_part.reserve(parts);
+    const unsigned blocks = grad_blocks(n);
+    parts = blocks * MWAVES;
+    partial.reserve((size_t)parts * PART_STRIDE);
     grad.reserve(MLP_NPARAM);
     loss.reserve(1);
-    k_mlp_grad<<<parts, 64 * MWAVES, 0, s>>>(theta, packed.get(), x, t, n, partial.get(), loss_part.get());
+    k_mlp_grad<<<blocks, 64 * MWAVES, 0, s>>>(theta, packed.get(), x, t, n, partial.get());
     SPH_HIP(hipGetLastError());
 }
 
 void MLPTrainer::loss_grad(hipStream_t s, const float *theta, const float *x, const float *t, unsigned n) {
     pack(s, theta);
     sums(s, theta, x, t, n);
-    k_mlp_grad_reduce<false><<<(MLP_NPARAM + 63) / 64, 64 * RSLICES, 0, s>>>(partial.get(), loss_part.get(), parts, n,
-                                                                           grad.get(), loss.get(), AdamArgs{});
+    k_mlp_grad_reduce<false><<<PART_STRIDE / REDUCE_COLS, REDUCE_THREADS, 0, s>>>(partial.get(), parts, n, grad.get(),
+                                                                                  loss.get(), AdamArgs{});
     SPH_HIP(hipGetLastError());
 }
 
-void MLPTrainer::start(hipStream_t s, const float *theta) {
+void MLPTrainer::start(hipStream_t s, const float *theta, unsigned n) {
     pack(s, theta);
+    partial.reserve((size_t)grad_blocks(n) * MWAVES * PART_STRIDE);
     adam_m.reserve(MLP_NPARAM);
     adam_v.reserve(MLP_NPARAM);
     fill_u32(s, reinterpret_cast<unsigned *>(adam_m.get()), MLP_NPARAM, 0u);
@@ -546,8 +535,8 @@ void MLPTrainer::step(hipStream_t s, float *theta, const float *x, const float *
     sums(s, theta, x, t, n);
     const AdamArgs a{theta, adam_m.get(), adam_v.get(), packed.get(), (float)std::pow(0.9, step),
                      (float)std::pow(0.999, step), lr};
-    k_mlp_grad_reduce<true><<<(MLP_NPARAM + 63) / 64, 64 * RSLICES, 0, s>>>(partial.get(), loss_part.get(), parts, n,
-                                                                          grad.get(), loss.get(), a);
+    k_mlp_grad_reduce<true><<<PART_STRIDE / REDUCE_COLS, REDUCE_THREADS, 0, s>>>(partial.get(), parts, n, grad.get(),
+                                                                                 loss.get(), a);
     SPH_HIP(hipGetLastError());
 }
 
@@ -619,7 +608,7 @@ int sph_mlp_train(float *theta, const float *x, const float *t, size_t n, int st
         k_gather_rows<<<nblocks(2 * n), BLOCK>>>(dorder.get(), n, ux.get(), ut.get(), dx.get(), dtt.get());
         SPH_HIP(hipGetLastError());
         MLPTrainer tr;
-        tr.start(nullptr, dt.get());
+        tr.start(nullptr, dt.get(), (unsigned)n);
         const size_t b = std::min<size_t>((size_t)batch, n);
         const size_t nbatches = std::max<size_t>(1, n / b);
         for (int it = 0; it < steps; it++) {

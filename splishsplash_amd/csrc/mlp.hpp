@@ -23,13 +23,14 @@ void mlp_forward(hipStream_t s, const float *theta, const float *x, unsigned n, 
 // respect to theta, and the loss (device pointers; scratch grows as needed).
 class MLPTrainer {
 public:
-    DBuf<float> partial, grad, loss_part, adam_m, adam_v, loss;
+    DBuf<float> partial, grad, adam_m, adam_v, loss;
     DBuf<short> packed;  // BF16 weights in operand order (see mlp.hip)
     unsigned parts = 0;
     void loss_grad(hipStream_t s, const float *theta, const float *x, const float *t, unsigned n);
-    // Adam from zero moments: start, then step 1, 2, ... on minibatches of n
-    // rows; theta changes only through step in between.
-    void start(hipStream_t s, const float *theta);
+    // Adam from zero moments: start (with the most rows that follow), then
+    // step 1, 2, ... on minibatches of n rows; theta changes only through
+    // step in between.
+    void start(hipStream_t s, const float *theta, unsigned n);
     void step(hipStream_t s, float *theta, const float *x, const float *t, unsigned n, int step, float lr);
 
 private:

@@ -84,3 +84,24 @@ def test_gradient_at_tile_and_block_edges(n):
     th, l0 = capi.mlp_train(theta, x, t, steps=0, batch=7, seed=3)
     np.testing.assert_array_equal(th, theta)
     assert l0 == pytest.approx(loss, rel=1e-5)
+
+
+@pytest.mark.parametrize("tiles", [2, 64, 512, 1024])
+def test_gradient_sums_are_taken_tile_by_tile(tiles):
+    # Up to 1,024 tiles of 32 rows a wave takes one each, and the gradients
+    # and losses of the tiles are added in FP32, one after the other: bit for
+    # bit, since 1 / n of a power of two only moves exponents.
+    n = 32 * tiles
+    rng = np.random.default_rng(tiles)
+    theta = M.init(4).astype(np.float32)
+    x = rng.normal(size=(n, 6)).astype(np.float32)
+    t = rng.normal(size=n).astype(np.float32)
+    loss, g = capi.mlp_loss_grad(theta, x, t)
+    go, lo = np.zeros_like(g), np.float32(0)
+    for k in range(0, n, 32):
+        l1, g1 = capi.mlp_loss_grad(theta, x[k:k + 32], t[k:k + 32])
+        go = go + g1 * np.float32(1 / tiles)
+        lo = lo + np.float32(l1) * np.float32(32)
+    assert g.dtype == np.float32
+    np.testing.assert_array_equal(g, go)
+    assert np.float32(loss) == lo / np.float32(n)

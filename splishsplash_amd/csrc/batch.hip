@@ -197,6 +197,9 @@ struct Group {
         std::vector<size_t> now;
         for (DFSPH *s : scenes) now.push_back(s->n());
         if (now == sizes && nbA) return;
+        for (DFSPH *s : scenes)
+            SPH_REQUIRE(2 * (size_t)nblocks(s->n() * (size_t)lanesJ) <= s->partial_room(), SPH_ERR_STATE,
+                        "batch: more error partials than the scene has room for");
         drop_graphs();
         sizes = now;
         const std::vector<uint4> a = block_map(now, lanesA), j = block_map(now, lanesJ);
@@ -250,13 +253,17 @@ struct BatchRunner {
 
     // Groups and block maps (once each scene's lanes are known).
     void setup(const std::vector<DFSPH *> &all) {
-        // group by the scenes' lanes
+        // group by the scenes' lanes: the same scenes at other lanes (a scene
+        // that has grown, or is stepped in other company) are another group
         std::map<std::pair<int, int>, std::vector<DFSPH *>> by;
         for (DFSPH *s : all) by[{s->lanes_accel(), s->lanes_jacobi()}].push_back(s);
         bool same = by.size() == groups.size();
         if (same) {
             size_t g = 0;
-            for (auto &kv : by) same = same && groups[g++]->scenes == kv.second;
+            for (auto &kv : by) {
+                const Group &h = *groups[g++];
+                same = same && h.scenes == kv.second && h.lanesA == kv.first.first && h.lanesJ == kv.first.second;
+            }
         }
         if (!same) {
             groups.clear();

@@ -211,6 +211,7 @@ public:
     int lanes_accel() const { return lppA_; }
     int lanes_jacobi() const { return lpp_; }
     Dev device_state() const { return dev(); }
+    size_t partial_room() const { return partial_.n; }  // reduction partials (doubles) a launch may write
     bool batchable() const;  // the plain DFSPH step with the reference's warm starts
     bool first_step_pending() const { return !picked_; }  // the next step sets up and picks the lanes per particle
     bool any_xsph() const;   // XSPH acts in some fluid model

@@ -194,6 +194,34 @@ def test_batch_first_steps_of_fresh_handles(mode):
         assert a.counters()["total_iterations"] == b.counters()["total_iterations"]
 
 
+@pytest.mark.parametrize("mode", ["batched", "graphs"])
+def test_batch_follows_scenes_that_change_lanes(mode):
+    # Up to 40,960 particles stepped together 16 lanes share a particle,
+    # beyond one lane takes it: scenes that grow past that between two calls
+    # on the same handles run at their new lanes. The FP64 error sums are
+    # grouped by the blocks of a launch, so they too are those of the scene
+    # alone only where the batch launches as many.
+    sc = scenes.dam_break_variant(11, per_side=27, aspect=3.0, n_spheres=0)
+    more = scenes.lattice_block((34, 27, 27), 0.05, (1.6, 0.1, 0.1))  # in the free part of the box
+    alone, batch = learned.make_sim(sc), learned.make_sim(sc)
+    capi.set_batch_mode(mode)
+    try:
+        for lanes in (16, 1):
+            if lanes == 1:
+                alone.emit_particles(more)
+                batch.emit_particles(more)
+            alone.step(3)
+            capi.step_batch([batch], 3)
+            assert alone.counters()["lanes_per_particle"] == batch.counters()["lanes_per_particle"] == lanes
+            for f in ("position", "velocity", "p / rho^2"):
+                np.testing.assert_array_equal(alone.get(f), batch.get(f), err_msg=f)
+            ca, cb = alone.counters(), batch.counters()
+            for c in ("total_iterations", "total_iterations_v", "avg_density_err", "avg_divergence_err", "time"):
+                assert ca[c] == cb[c], c
+    finally:
+        capi.set_batch_mode("auto")
+
+
 @pytest.mark.parametrize("mode", ["threads", "batched", "graphs", "auto"])
 def test_batch_step_matches_scene_by_scene(mode):
     # Scenes stepped together give the same results as each stepped alone,

@@ -47,6 +47,7 @@ __global__ __launch_bounds__(BLOCK) void k_permute_fluid(const unsigned *__restr
         C->maxcnt_f = 0;
         C->maxcnt_b = 0;
         C->ovf16 = 0;
+        C->tiles_over = 0;
     }
     if (k >= n) return;
     const unsigned j = perm[k];
@@ -174,19 +175,20 @@ __device__ __forceinline__ void fluid_pairs(const Dev &D, unsigned i, unsigned h
 // were). Consecutive particles share most of their neighbours, so a tile of
 // 256 needs about 8 slots a particle instead of 30: a tiled sweep copies
 // those to LDS once, coalesced, and its pairs read LDS. At 1M particles
-// (pressure / divergence iterations) k_accel 47 / 44 -> 28 / 36 us, k_jacobi
-// 73 / 65 -> 52 / 47 us; at 69k 9.3 / 10.0 -> 8.1 / 9.6 and 14.8 / 14.0 ->
-// 12.2 / 11.4 us. They are now bound by the vector instructions, 45 a pair,
-// some 12 % of them in the FP64 band of table_step. Tiles of 128 particles
+// (pressure / divergence iterations) k_accel 44 / 48 -> 28 / 35 us, k_jacobi
+// 69 / 73 -> 50 / 53 us; at 176k 15 / 14 -> 12 / 14 and 20 / 18 -> 17 / 15 us.
+// They are now bound by the vector instructions, 45 a pair, some 12 % of them
+// in the FP64 band of table_step. Tiles of 128 particles
 // take as long in the sweeps and half as long again to build.
 //
 // k_tile_lists, once a step: marks the tile's neighbour slots in a bitmap of
 // the 65536 slots around the tile, numbers the marked ones in slot order and
 // rewrites the packed lists with these numbers, entries in the same order
-// (86 us at 1M particles, 31 us at 69k; bound by LDS: a marked slot is an
+// (85 us at 1M particles, 33 us at 111k; bound by LDS: a marked slot is an
 // atomic, a rewritten one two reads).
 // A tile with more than TILE_CAP slots, or slots outside the window, keeps a
-// count of zero and its sweeps read memory as before.
+// count of zero, its sweeps read memory as before, and the control block
+// counts it.
 constexpr unsigned TILE_WORDS = 65536 / 32;
 __global__ __launch_bounds__(TILE) void k_tile_lists(Dev D, uint4 *__restrict__ nt16,
                                                      unsigned *__restrict__ tslot, unsigned *__restrict__ tcount) {
@@ -248,6 +250,7 @@ __global__ __launch_bounds__(TILE) void k_tile_lists(Dev D, uint4 *__restrict__ 
     }
     const bool fits = total <= TILE_CAP && bad == 0u;
     if (t == 0) tcount[blk] = fits ? total : 0u;
+    if (t == 0 && !fits) atomicAdd(&D.ctl->tiles_over, 1u);
     if (!fits) return;
     short *const out = reinterpret_cast<short *>(tslot + (size_t)blk * (TILE_CAP / 2));
 #pragma unroll
@@ -315,45 +318,36 @@ __device__ __forceinline__ void tile_stage(const Dev &D, unsigned blk, unsigned 
 // first are loaded before the tile is staged. (Words loaded where they are
 // used: k_accel 43 / 51 us, k_jacobi 61 / 58 us at 1M particles.)
 template <int LPP> struct TileWords {
-    static constexpr int W = 4 / LPP;  // words of a quad per lane
-    typedef unsigned Quad __attribute__((ext_vector_type(W == 1 ? 2 : W)));  // (one word: .x)
+    static constexpr int W = 4 / LPP;  // words of a quad per lane: 4 or 2
+    typedef unsigned Quad __attribute__((ext_vector_type(W)));
     Quad c, n, m;
     const unsigned *P;
-    __device__ __forceinline__ static Quad load(const unsigned *p) {
-        if constexpr (W == 1)
-            return Quad{*p, 0u};
-        else
-            return *reinterpret_cast<const Quad *>(p);
-    }
-    __device__ __forceinline__ TileWords(const Dev &D, unsigned i, unsigned hl)
-        : P(D.nt16 + 4 * (size_t)i + (LPP == 4 ? ((hl & 1u) << 1 | hl >> 1) : W * hl)) {
+    __device__ __forceinline__ static Quad load(const unsigned *p) { return *reinterpret_cast<const Quad *>(p); }
+    __device__ __forceinline__ TileWords(const Dev &D, unsigned i, unsigned hl) : P(D.nt16 + 4 * (size_t)i + W * hl) {
         const size_t S = 4 * (size_t)D.stride;
         const unsigned last = D.quads16 - 1u;
         const bool act = i < D.n;
         c = act ? load(P) : Quad{};
         n = act ? load(P + (last < 1u ? last : 1u) * S) : Quad{};
-        m = act && W < 4 ? load(P + (last < 2u ? last : 2u) * S) : Quad{};
+        m = act && W == 2 ? load(P + (last < 2u ? last : 2u) * S) : Quad{};
     }
     template <class F> __device__ __forceinline__ void pairs(const Dev &D, unsigned hl, unsigned cnt, F &&f) {
-        constexpr unsigned AHEAD = W < 4 ? 3 : 2;
+        constexpr unsigned AHEAD = W == 2 ? 3 : 2;
         const size_t S = 4 * (size_t)D.stride;
         const unsigned full = cnt >> 1, quads = (cnt + 7u) >> 3;  // words of two neighbours; quads
         const unsigned *p = P + AHEAD * S;
         unsigned w = hl, k = AHEAD;
         auto four = [&](unsigned a, unsigned b) { f(a & 0xffffu, a >> 16, b & 0xffffu, b >> 16); };
-        auto two = [&](unsigned a) { f(a & 0xffffu, a >> 16); };
         for (; w + (W - 1) * LPP < full; w += 4, k++, p += S) {
             const Quad q = c;
             c = n;
-            if (W < 4) n = m;
-            if (k < quads) (W < 4 ? m : n) = load(p);
+            if (W == 2) n = m;
+            if (k < quads) (W == 2 ? m : n) = load(p);
             if constexpr (W == 4) {
                 four(q.x, q[2]);
                 four(q.y, q[3]);
-            } else if constexpr (W == 2) {
-                four(q.x, q.y);
             } else {
-                two(q.x);
+                four(q.x, q.y);
             }
         }
         // the lane's rest of c: fewer than W full words, and the odd entry
@@ -365,12 +359,11 @@ template <int LPP> struct TileWords {
                 c[2] = c[3];
                 w += 2;
             }
-        if constexpr (W > 1)
-            if (w < full) {
-                two(a);
-                a = c[W / 2];
-                w += LPP;
-            }
+        if (w < full) {
+            f(a & 0xffffu, a >> 16);
+            a = c[W / 2];
+            w += LPP;
+        }
         if ((cnt & 1u) && w == full) f(a & 0xffffu);
     }
 };
@@ -2778,6 +2771,7 @@ void DFSPH::upload_ctl_field(size_t off, const void *src, size_t bytes) {
 // Per-particle device buffers for stride_ slots (contents not preserved).
 void DFSPH::alloc_particles() {
     const size_t S = stride_;
+    no_tile_room_ = false;
     SPH_REQUIRE(S <= GATHER_MAX, SPH_ERR_RANGE, "at most 2^28 particle slots per time step");
     for (DBuf<float4> *b : {&x_, &v_, &v2_, &a_, &ap_, &vdiff_, &xc_, &x2_, &vdiff2_, &xc2_}) b->reserve(S);
     const size_t nobj = maps() ? vm_shapes_.size() : 0;
@@ -3008,34 +3002,67 @@ void DFSPH::build_lists() {
     use16_ = hctl_->ovf16 == 0u;
     lists_max_ = hctl_->maxcnt_f;
     tiled_ = tiles_known_ = false;
+    list_its_ = 0;
+    // how many tiles were overfull counts for the next 16 lists
+    if (tiles_over_ && ++tiles_wait_ > 16) tiles_over_ = 0;
     lists_n_ = n_;
     have_lists_ = true;
 }
 
+// Whether tiles gain more in the iterations on these lists than they cost.
+// At n particles the two tiled sweeps of an iteration save about 35 ps n -
+// 2.5 us and the tiles take 27 us + 60 ps n (measured / formula, us, 1 or 2
+// lanes: 111k saved 2.0-3.4 / 1.4, built 33 / 34; 176k 3.4-6.6 / 3.6, 35 /
+// 38; 262k 6.0-8.7 / 6.7, 38 / 43; 593k 15-20 / 18, 59 / 63; 1M 31-34 / 33,
+// 85 / 87; 2M 56-77 / 68, 158 / 147): they pay from 3 iterations on at 1M, 10
+// at 176k, 25 at 111k. Expected are the iterations of the last solves, or as
+// many again as the lists have already seen. An overfull tile is taken to
+// lose what another saves: its blocks gather beside LDS that they do not use
+// (62-64 % of the tiles overfull, us an iteration gathered / tiled: 133k 57 /
+// 63, 293k 94 / 98, 547k 159 / 150). Four lanes read tiles no faster than
+// memory (1M: 124 us an iteration, 126 gathered), and below SMALL_PARTICLES
+// the 16 ordered lanes hide the latency that staging would add.
+bool DFSPH::tiles_pay() const {
+    const double n = (double)n_, its = std::max(lastIt_ + (P.enable_divergence_solver ? lastItV_ : 0), list_its_);
+    const double fit = 1.0 - 2.0 * tiles_over_ * TILE / n;
+    return its * fit * (0.035 * n - 2500.0) >= 27000.0 + 0.06 * n;  // ns
+}
+
 // The lists of the iterations' sweeps (single-model scenes whose lists are
-// packed), from SMALL_PARTICLES on: there a step's dozen or
-// more iterations save 3 us each and the tiles cost 31 us, at 166k 5 against
-// 35, at 1M 45 against 86. Below it the 16 ordered lanes hide the latency
-// that staging would add.
-// They are built when the first iteration asks for them: a search, a density
-// or a batched solve has no use for them.
+// packed), built when an iteration asks for them and they pay: a search, a
+// density or a batched solve has no use for them.
 void DFSPH::build_tiles() {
     if (tiles_known_) return;
+    const bool can = have_lists_ && lists_n_ == n_ && use16_ && !models_ && method_ == SPH_METHOD_DFSPH &&
+                     n_ >= SMALL_PARTICLES && lpp_ <= 2 && lppA_ <= 2 && !no_tile_room_;
+    if (can && !tiles_pay()) return;
     tiles_known_ = true;
-    tiled_ = have_lists_ && lists_n_ == n_ && use16_ && !models_ && method_ == SPH_METHOD_DFSPH && n_ >= SMALL_PARTICLES;
-    if (!tiled_) return;
+    if (!can) return;
     const unsigned nt = ((unsigned)n_ + TILE - 1) / TILE;
-    nt16_.reserve(4 * (size_t)((capF_ + 7) / 8) * stride_);
-    tslot_.reserve((size_t)nt * (TILE_CAP / 2));
-    tcount_.reserve(nt);
+    try {
+        nt16_.reserve(4 * (size_t)((capF_ + 7) / 8) * stride_);
+        tslot_.reserve((size_t)nt * (TILE_CAP / 2));
+        tcount_.reserve(nt);
+    } catch (const Error &e) {
+        if (e.code != SPH_ERR_OOM) throw;
+        // the sweeps gather, until the particles' buffers change size
+        (void)hipGetLastError();
+        nt16_.release();
+        tslot_.release();
+        tcount_.release();
+        no_tile_room_ = true;
+        return;
+    }
+    tiled_ = true;
+    tiles_wait_ = 0;
     TimedScope ts(timer, stream, "tile_lists");
     k_tile_lists<<<nt, TILE, 0, stream>>>(dev(), reinterpret_cast<uint4 *>(nt16_.get()), tslot_.get(), tcount_.get());
     SPH_HIP(hipGetLastError());
 }
 
-// Lanes per particle of a small count. The two give the same
-// sums bit for bit, so the rule only weighs time: shared pairs hide the
-// memory latency of a nearly idle GPU and cost three times the instructions.
+// Lanes per particle of a small count. The two give the same sums
+// bit for bit, so the rule only weighs time: shared pairs hide the memory
+// latency of a nearly idle GPU and cost three times the instructions.
 // Whole steps (us), one lane / shared, Akinci walls and plain start: 2,197
 // particles 550 / 407, 12,167 particles 895 / 687, 32,768 particles 1307 /
 // 1203, 50,653 particles 1335 / 1425. Eight scenes of 20k-80k particles
@@ -3247,8 +3274,8 @@ static void launch_iteration_sweep(int lanes, unsigned n, hipStream_t s, const D
         else                                                                      \
             k_accel_tile<PRESSURE, L><<<nb, TILE * L, 0, s>>>(D, check_done);     \
     }
-    if (D.nt16 && lanes <= 4) {
-        SWEEP(1) SWEEP(2) SWEEP(4)
+    if (D.nt16 && lanes <= 2) {
+        SWEEP(1) SWEEP(2)
         SPH_HIP(hipGetLastError());
     } else {
         launch_sweep<PRESSURE, JACOBI>(lanes, n, s, D, check_done);
@@ -3279,6 +3306,7 @@ void DFSPH::iteration_any(bool force) {
         return;
     }
     build_tiles();
+    list_its_++;
     const Dev D = dev();
     {
         TimedScope ts(timer, stream, PRESSURE ? "pressure_accel" : "pressure_accel_v");
@@ -3783,6 +3811,7 @@ int DFSPH::run_solver(bool pressure, int already, bool copy_w) {
                 div_iteration(false);
         }
         read_ctl();
+        if (tiled_) tiles_over_ = hctl_->tiles_over;
         const int done = pressure ? hctl_->done : hctl_->done_v;
         if (done || launched >= maxIt) break;
         // past the predicted count: two iterations per round trip (an

@@ -33,6 +33,7 @@ struct Ctl {
     int flags;         // bit0: non-finite value in a reduction
     unsigned maxcnt_f, maxcnt_b;
     unsigned ovf16;               // a packed list difference did not fit
+    unsigned tiles_over;          // tiles that keep no slots (see k_tile_lists)
     double kref, kref_v;          // stiffness scales of the learned start
     unsigned nlearn, nlearn_v;    // particles that kept the learned start
     unsigned nsamp, nsamp_v;      // training samples written
@@ -51,14 +52,14 @@ struct Dev {
     // the low and high halves of nf16[w * stride + i]. The solver sweeps read
     // these -- half the index bytes and index loads of nf.
     const unsigned *nf16;
-    // Tiled lists (null below SMALL_PARTICLES and where nf16 is): the union
+    // Tiled lists (null where nf16 is and unless they pay): the union
     // of the neighbours of particles b TILE .. b TILE + TILE - 1, tcount[b]
     // slots (0: more than TILE_CAP, or too far apart), as int16 differences
     // slot - b TILE, two per word, at tslot[b TILE_CAP / 2]; and the lists
     // of those particles as 16-bit places in the union, the words of nf16 by
     // quads: words 4g, 4g + 2, 4g + 1, 4g + 3 of particle i at
-    // nt16[4 (g stride + i)], g < quads16. One, two or four lanes of the
-    // particle then each load their share of a quad at once.
+    // nt16[4 (g stride + i)], g < quads16. One or two lanes of the particle
+    // then each load their share of a quad at once.
     const unsigned *nt16, *tslot, *tcount;
     unsigned quads16;
     const float4 *bx;  // Akinci particles (x, y, z, volume), cell-sorted
@@ -314,6 +315,10 @@ private:
     size_t lists_n_ = 0;     // particles the current lists were built for
     unsigned lists_max_ = 0;  // the longest of them
     bool tiles_known_ = false;  // whether they do has been settled for these lists
+    int list_its_ = 0;       // solver iterations on the current lists
+    unsigned tiles_over_ = 0, tiles_wait_ = 0;  // overfull tiles when last built, lists since
+    bool no_tile_room_ = false;  // their allocation failed at this capacity
+    bool tiles_pay() const;
     void build_tiles();
     void ensure_pair_grad();
     DBuf<float4> minv_, cgx_, cgr_, cgp_, cgz_, cgt_;

@@ -9,9 +9,10 @@ import os
 
 import numpy as np
 import pytest
+from scipy.spatial import cKDTree
 
 from oracle import oracle
-from splishsplash_amd import capi, scenes
+from splishsplash_amd import capi, learned, scenes
 from splishsplash_amd.params import BOUNDARY_BENDER2019, BOUNDARY_NONE, VISCOSITY_STANDARD, VISCOSITY_WEILER2018, default_params
 
 pytestmark = pytest.mark.gpu
@@ -217,52 +218,90 @@ def test_lanes_of_long_lists_follow_their_rule():
         assert (c["lanes_per_particle"], c["lanes_per_particle_accel"]) == lanes
 
 
-@pytest.mark.parametrize("lanes", [1, 2, 4])
-def test_tiled_sweeps_match_gathered_ones(lanes):
-    # From 65,536 particles on the iterations read neighbours from tiles in
-    # LDS. The same scene with 300 more points in one spot far away keeps no
-    # packed lists, hence no tiles, and gathers. 70,411 particles leave the
-    # last tile ragged, particles strewn alone have no neighbours, and tiles
-    # across thin dense sheets outgrow their share of LDS. With one lane per
-    # particle both take the same sums, bit for bit; with more the gathered
-    # lists are split differently: two orders of at most 128 terms, each
-    # within 127 2^-24 of the terms' absolute sum, which stays below 32 times
-    # the largest result.
-    sc = scenes.dam_break_small(per_side=(44, 40, 38))
-    sheet = scenes.lattice_block((1, 30, 30), 0.02, (2.4, 0.1, 0.1), jitter=0.0005, seed=4)
-    dense = np.concatenate([sheet + np.float32([0.21 * k, 0, 0]) for k in range(7)])
-    alone = scenes.f32([[3.9, 0.1 + 0.15 * k, 1.9] for k in range(11)])
-    x = np.concatenate([sc["x"][:70400 - len(dense)], dense, alone])
-    n = len(x)
-    assert n == 70411
-    spot = np.float32([3.2, 2.6, 1.2]) + np.random.default_rng(8).uniform(-0.01, 0.01, (300, 3)).astype(np.float32)
-    v, p, pv = perturbed_state(x, seed=11)
-    out = []
-    for extra in (np.zeros((0, 3), np.float32), spot):
-        g = capi.TimeStepDFSPH(sc["params"])
-        g.set_fluid(scenes.f32(np.concatenate([x, extra])), scenes.f32(np.concatenate([v, 0 * extra])))
-        g.add_boundary_particles(sc["boundary_x"])
+def tile_unions(x, h, lo):
+    """Per 256 consecutive particles in cell order (rows of z and y, quarter
+    cells along x, the grid's origin two supports and a cell below lo): how
+    many particles are neighbours of one of them."""
+    cell = h * (1 + 1e-4)
+    c = np.floor((x - (np.asarray(lo) - 2 * h - cell)) / cell * [4, 1, 1]).astype(np.int64)
+    order = np.lexsort((c[:, 0], c[:, 1], c[:, 2]))
+    lists = cKDTree(x.astype(np.float64)).query_ball_point(x[order].astype(np.float64), h)
+    return np.array([len({j for i, near in zip(order[b:b + 256], lists[b:b + 256]) for j in near if j != i})
+                     for b in range(0, len(x), 256)])
+
+
+@pytest.mark.parametrize("walls", ["akinci", "bender"])
+@pytest.mark.parametrize("lanes", [1, 2])
+def test_tiled_iterations_match_gathered_ones(walls, lanes):
+    # Whole steps of a scene alone, whose iterations read neighbours from
+    # tiles in LDS, against the same scene in a batched solve, which gathers
+    # from the same packed lists: bit for bit. Compressed to 0.85 of its
+    # spacing the long block has tiles that fit their share of LDS and tiles
+    # that do not; 133,771 particles leave the last one ragged, and particles
+    # strewn alone have no neighbours.
+    sc = scenes.dam_break_small(boundary=walls, max_error=0.001, max_error_v=0.01, viscosity_method=VISCOSITY_STANDARD,
+                                viscosity=0.01)
+    block = scenes.lattice_block((88, 40, 38), 0.0425, (0.1, 0.1, 0.1), jitter=0.001, seed=1)
+    alone = scenes.f32([[3.95, 2.2 + 0.05 * (k % 2), 0.1 + 0.15 * k] for k in range(11)])
+    x = scenes.f32(np.concatenate([block, alone]))
+    assert len(x) == 133771
+    over = np.count_nonzero(tile_unions(x, 0.1, (0.0, 0.0, 0.0)) > 1856)
+    assert 100 < over < 200  # of 523 tiles
+    sims = []
+    for batched in (False, True):
+        g = learned.make_sim(dict(sc, x=x, v=np.zeros_like(x)))
         g.set_lanes_per_particle(lanes)
         g.enable_timing()
-        g.init()
+        capi.set_batch_mode("batched")
+        try:
+            if batched:
+                capi.step_batch([g], 3)
+            else:
+                g.step(3)
+        finally:
+            capi.set_batch_mode("auto")
+        sims.append(g)
+    a, b = sims
+    assert "tile_lists" in a.kernel_stats() and "tile_lists" not in b.kernel_stats()
+    for f in ("position", "velocity", "p / rho^2", "p_v / rho^2", "pressure acceleration"):
+        assert np.isfinite(a.get(f)).all()
+        np.testing.assert_array_equal(a.get(f), b.get(f), err_msg=f)
+    ca, cb = a.counters(), b.counters()
+    for c in ("total_iterations", "total_iterations_v", "avg_density_err", "avg_divergence_err", "time"):
+        assert ca[c] == cb[c], c
+
+
+def test_tiles_are_built_once_the_iterations_pay_for_them():
+    # At 120,384 particles tiles pay from 20 iterations on one list; the
+    # last solves' counts are 3 for a new handle.
+    x = scenes.lattice_block((76, 44, 36), 0.05, (0.1, 0.1, 0.1), jitter=0.001, seed=1)
+    g = capi.TimeStepDFSPH(default_params(boundary_handling_method=BOUNDARY_NONE))
+    g.set_fluid(x)
+    g.enable_timing()
+    for _ in range(2):
         g.stage("neighborhood_search")
-        pad = lambda a: scenes.f32(np.concatenate([a, np.zeros(len(extra), np.float32)]))
-        g.set("p / rho^2", pad(p))
-        g.set("p_v / rho^2", pad(pv))
-        got = {}
-        for stage in ("densities", "dfsph_factor", "divergence_setup", "divergence_iter", "pressure_setup", "pressure_iter",
-                      "pressure_iter"):
+        g.stage("densities")
+        g.stage("dfsph_factor")
+        g.stage("pressure_setup")
+        for _ in range(20):
+            g.stage("pressure_iter")
+        assert "tile_lists" not in g.kernel_stats()
+    g.stage("pressure_iter")
+    assert g.kernel_stats()["tile_lists"][0] == 1
+
+
+def test_tiles_that_are_mostly_overfull_wait():
+    # At 0.8 of its spacing 324 of the block's 520 tiles outgrow their share
+    # of LDS: after one solve the next 16 lists go without tiles.
+    sc = scenes.dam_break_small(boundary="bender")
+    x = scenes.lattice_block((95, 40, 35), 0.04, (0.1, 0.1, 0.1), jitter=0.001, seed=1)
+    assert 300 < np.count_nonzero(tile_unions(x, 0.1, (0.0, 0.0, 0.0)) > 1856) < 350
+    g = learned.make_sim(dict(sc, x=x, v=np.zeros_like(x)))
+    g.enable_timing()
+    for k in range(18):
+        for stage in ("neighborhood_search", "volume_maps", "densities", "dfsph_factor", "pressure_solve"):
             g.stage(stage)
-            for f in ("pressure acceleration", "p / rho^2", "p_v / rho^2"):
-                got[stage, f] = g.get(f)[:n]
-        assert ("tile_lists" in g.kernel_stats()) == (len(extra) == 0)
-        out.append(got)
-    for k, a in out[0].items():
-        b = out[1][k]
-        if lanes == 1:
-            np.testing.assert_array_equal(a, b, err_msg=str(k))
-        else:
-            np.testing.assert_allclose(a, b, rtol=0, atol=2 * 127 * 2.0**-24 * 32 * np.abs(b).max(), err_msg=str(k))
+        assert g.kernel_stats()["tile_lists"][0] == (1 if k < 17 else 2)
 
 
 def vm_scene(n=16, corner=0.06):

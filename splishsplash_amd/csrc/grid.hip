@@ -583,10 +583,11 @@ __global__ __launch_bounds__(BLOCK) void k_csr_wave(const float4 *__restrict__ q
                                                     const unsigned *__restrict__ srcmap,
                                                     const unsigned *__restrict__ start, GridDesc g, float r2,
                                                     float r2t, const unsigned *__restrict__ rowoff,
-                                                    unsigned *__restrict__ out, unsigned *__restrict__ cnt) {
+                                                    unsigned *__restrict__ out, unsigned *__restrict__ cnt, unsigned w0) {
     const unsigned lane = threadIdx.x & 63u;
-    const unsigned w = __builtin_amdgcn_readfirstlane(xcd_block() * (BLOCK / 64) + (threadIdx.x >> 6));
-    if (w >= nq) return;
+    const unsigned wl = __builtin_amdgcn_readfirstlane(xcd_block() * (BLOCK / 64) + (threadIdx.x >> 6));
+    if (wl >= nq - w0) return;
+    const unsigned w = w0 + wl;
     const float4 xi = q[w];
     const unsigned i = qmap ? qmap[w] : w;
     unsigned sv = 0u, ev = 0u;
@@ -851,6 +852,10 @@ void build_lists_colmajor(hipStream_t s, const float4 *q, unsigned nq, const flo
 // (K = 34) 698 / 438 us: few lanes per SIMD leave the memory latency open,
 // and a wave per query issues about four times the instructions.
 constexpr unsigned CSR_WAVE_MAX = 1u << 17;
+// Queries of one launch with a wave each, of the `left` that remain: a launch
+// holds fewer than 2^32 threads. (Waves that take several queries in turn are
+// slower: 100k uniform points 235 -> 285 us.)
+unsigned csr_wave_slice(unsigned left) { return std::min(left, 1u << 25); }
 
 void build_lists_csr(hipStream_t s, const float4 *q, const unsigned *qmap, unsigned nq, const float4 *src,
                      unsigned nsrc, const unsigned *srcmap, const unsigned *start, const GridDesc &g, double radius, bool same_set,
@@ -860,20 +865,22 @@ void build_lists_csr(hipStream_t s, const float4 *q, const unsigned *qmap, unsig
     const float r2t = (float)(radius * radius * (1.0 + 1e-5));  // row trimming reach, as in build_lists_colmajor
     // (the lanes' buffer loads address 2^28 sources)
     const bool wave = nq < CSR_WAVE_MAX || nsrc >= GATHER_MAX;
-    const unsigned nb = wave ? nblocks((size_t)nq * 64) : nblocks(nq);
-#define CSR(K, SAME, FILL)                                                                                    \
-    K<SAME, FILL><<<nb, BLOCK, 0, s>>>(q, qmap, nq, src, nsrc, srcmap, start, g, r2, r2t, rowoff, out, cnt)
-#define CSR_SF(K)                                                          \
-    do {                                                                   \
-        if (same_set && rowoff) CSR(K, true, true);                        \
-        if (same_set && !rowoff) CSR(K, true, false);                      \
-        if (!same_set && rowoff) CSR(K, false, true);                      \
-        if (!same_set && !rowoff) CSR(K, false, false);                    \
+#define CSR(K, nb, SAME, FILL, ...) \
+    K<SAME, FILL><<<nb, BLOCK, 0, s>>>(q, qmap, nq, src, nsrc, srcmap, start, g, r2, r2t, rowoff, out, cnt, ##__VA_ARGS__)
+#define CSR_SF(K, nb, ...)                                                             \
+    do {                                                                               \
+        if (same_set && rowoff) CSR(K, nb, true, true, ##__VA_ARGS__);                 \
+        if (same_set && !rowoff) CSR(K, nb, true, false, ##__VA_ARGS__);               \
+        if (!same_set && rowoff) CSR(K, nb, false, true, ##__VA_ARGS__);               \
+        if (!same_set && !rowoff) CSR(K, nb, false, false, ##__VA_ARGS__);             \
     } while (0)
     if (wave)
-        CSR_SF(k_csr_wave);
+        for (unsigned w0 = 0, n; w0 < nq; w0 += n) {
+            n = csr_wave_slice(nq - w0);
+            CSR_SF(k_csr_wave, nblocks((size_t)n * 64), w0);
+        }
     else
-        CSR_SF(k_csr_lanes);
+        CSR_SF(k_csr_lanes, nblocks(nq));
 #undef CSR_SF
 #undef CSR
     SPH_HIP(hipGetLastError());

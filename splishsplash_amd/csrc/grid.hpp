@@ -100,6 +100,9 @@ void build_lists_colmajor(hipStream_t s, const float4 *q, unsigned nq, const flo
                           unsigned *cnt, unsigned *maxcnt, KernelTimer &T, const char *name,
                           unsigned *nbr16 = nullptr, unsigned *ovf16 = nullptr);
 
+// Queries that one launch with a wave per query takes of `left`.
+unsigned csr_wave_slice(unsigned left);
+
 // CSR variant for the drop-in search: sources cell-sorted with srcmap[slot] =
 // caller index of the source point, queries q with qmap[k] = caller index of
 // query k (null: k itself), best in cell order too. With rowoff == nullptr

@@ -78,3 +78,17 @@ def test_struct_layouts_agree_with_the_header():
         out = [int(v) for v in subprocess.run([exe], check=True, capture_output=True, text=True).stdout.split()]
     assert out[0] == ctypes.sizeof(DFSPHParams) and out[1] == ctypes.sizeof(DFSPHCounters)
     assert out[2:] == [getattr(DFSPHCounters, f).offset for f in fields]
+
+
+def test_wave_per_query_launches_stay_below_the_thread_limit():
+    # A launch holds fewer than 2^32 threads. With sources beyond 2^28 a wave
+    # takes a query at any count: 64 threads for each of 2^26 would pass it.
+    from splishsplash_amd import capi
+    take = capi.lib()["_ZN3sph14csr_wave_sliceEj"]
+    take.restype = ctypes.c_uint
+    for nq in (1, (1 << 25) - 1, 1 << 25, (1 << 25) + 1, 1 << 26, (1 << 28) + 1, (1 << 32) - 1):
+        left = nq
+        while left:
+            n = take(ctypes.c_uint(left))
+            assert 0 < n <= left and (64 * n + 255) // 256 * 256 < 1 << 32
+            left -= n

@@ -216,11 +216,11 @@ def expected_csr(x, radius, y=None):
     return off, idx[order]
 
 
-@pytest.mark.parametrize("n,knot", [(1, 0), (63, 0), (65, 40), (700, 700), (5003, 900), (131071, 0), (131072, 0),
-                                    (131109, 1500)])
+@pytest.mark.parametrize("n,knot", [(1, 0), (63, 0), (65, 40), (700, 700), (5003, 900), (65536, 0), (65537, 0),
+                                    (131071, 0), (131072, 0), (131109, 1500)])
 def test_drop_in_lists_keep_their_order(n, knot):
-    """Sizes around a wave and around the switch between a wave and a lane
-    per query; `knot` points crowd into a corner of one cell, so that rows
+    """Sizes around a wave, around the first query that a wave takes beside
+    another and around the switch between a wave and a lane per query; `knot` points crowd into a corner of one cell, so that rows
     hold far more candidates than one window or hit word."""
     rng = np.random.default_rng(n)
     x = rng.uniform(0.0, 1.0, (n, 3)).astype(np.float32)

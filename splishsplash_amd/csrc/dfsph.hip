@@ -1117,7 +1117,7 @@ __global__ __launch_bounds__(TILE *LPP) void k_jacobi_tile(Dev D, int check_done
 }
 
 template <bool PRESSURE, int LPP>
-__global__ __launch_bounds__(BLOCK, LPP == 2 ? 7 : 1) void k_jacobi(Dev D, int check_done) {
+__global__ __launch_bounds__(BLOCK) void k_jacobi(Dev D, int check_done) {
     jacobi_sweep<PRESSURE, LPP>(D, xcd_block(), blockIdx.x, check_done);
 }
 

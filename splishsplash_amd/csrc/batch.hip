@@ -128,8 +128,12 @@ unsigned xcd_range(unsigned b, unsigned B) {
 // batched launch = (scene, particle block, partial-sum slot). The particle
 // blocks of all scenes, concatenated, are spread over the XCDs as one
 // launch's would be (contiguous ranges per XCD); the slot is the hardware
-// block that takes the same particle block in the scene's own launch, so the
-// error partials, and with them every result, equal the scene's own.
+// block that takes the same particle block in the scene's own launch at these
+// lanes, so the error partials, and with them every result, equal the scene's
+// own. (A scene that takes 16 lanes alone and one in company has the same
+// neighbour sums, but FP64 partials over 16 particles a block instead of 256:
+// their totals, which decide when a solve ends and scale the CG's steps, may
+// differ in the last bit.)
 // With ids, entry k of n is scene ids[k] of the group's table (a map over
 // a subset of the scenes).
 std::vector<uint4> block_map(const std::vector<size_t> &n, int lanes, const std::vector<unsigned> *ids = nullptr) {

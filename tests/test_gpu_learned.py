@@ -222,6 +222,32 @@ def test_batch_follows_scenes_that_change_lanes(mode):
         capi.set_batch_mode("auto")
 
 
+@pytest.mark.parametrize("mode", ["threads", "graphs"])
+def test_batch_in_larger_company_keeps_the_fields(mode):
+    # Each scene takes 16 lanes per particle alone; together they are more
+    # than 40,960 particles and take one. Neighbour sums keep their order, so
+    # fields and iteration counts stay (only FP64 totals are grouped
+    # differently, in their last bits).
+    scs = [scenes.dam_break_variant(20 + k, per_side=(26, 27, 28)[k], n_spheres=k) for k in range(3)]
+    alone, batch = [learned.make_sim(sc) for sc in scs], [learned.make_sim(sc) for sc in scs]
+    assert max(sim.n for sim in alone) <= 40960 < sum(sim.n for sim in alone)
+    for sim in alone:
+        sim.step(8)
+    capi.set_batch_mode(mode)
+    try:
+        capi.step_batch(batch, 8)
+    finally:
+        capi.set_batch_mode("auto")
+    for a, b in zip(alone, batch):
+        ca, cb = a.counters(), b.counters()
+        assert (ca["lanes_per_particle"], cb["lanes_per_particle"]) == (16, 1)
+        for f in ("position", "velocity", "p / rho^2", "velocity difference"):
+            np.testing.assert_array_equal(a.get(f), b.get(f), err_msg=f)
+        assert ca["total_iterations"] == cb["total_iterations"]
+        assert ca["total_iterations_v"] == cb["total_iterations_v"]
+        assert ca["avg_density_err"] == pytest.approx(cb["avg_density_err"], rel=1e-12)
+
+
 @pytest.mark.parametrize("mode", ["threads", "batched", "graphs", "auto"])
 def test_batch_step_matches_scene_by_scene(mode):
     # Scenes stepped together give the same results as each stepped alone,

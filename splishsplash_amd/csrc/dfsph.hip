@@ -3015,15 +3015,16 @@ void DFSPH::build_lists() {
 // lanes: 111k saved 2.0-3.4 / 1.4, built 33 / 34; 176k 3.4-6.6 / 3.6, 35 /
 // 38; 262k 6.0-8.7 / 6.7, 38 / 43; 593k 15-20 / 18, 59 / 63; 1M 31-34 / 33,
 // 85 / 87; 2M 56-77 / 68, 158 / 147): they pay from 3 iterations on at 1M, 10
-// at 176k, 25 at 111k. Expected are the iterations of the last solves, or as
-// many again as the lists have already seen. An overfull tile is taken to
+// at 176k, 25 at 111k. Expected are the iterations of the last solves, or half
+// as many again as the lists have already seen (a solve that ends near the
+// last one's count is not worth tiles at its end). An overfull tile is taken to
 // lose what another saves: its blocks gather beside LDS that they do not use
 // (62-64 % of the tiles overfull, us an iteration gathered / tiled: 133k 57 /
 // 63, 293k 94 / 98, 547k 159 / 150). Four lanes read tiles no faster than
 // memory (1M: 124 us an iteration, 126 gathered), and below SMALL_PARTICLES
 // the 16 ordered lanes hide the latency that staging would add.
 bool DFSPH::tiles_pay() const {
-    const double n = (double)n_, its = std::max(lastIt_ + (P.enable_divergence_solver ? lastItV_ : 0), list_its_);
+    const double n = (double)n_, its = std::max(lastIt_ + (P.enable_divergence_solver ? lastItV_ : 0), list_its_ / 2);
     const double fit = 1.0 - 2.0 * tiles_over_ * TILE / n;
     return its * fit * (0.035 * n - 2500.0) >= 27000.0 + 0.06 * n;  // ns
 }

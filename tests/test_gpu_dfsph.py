@@ -272,8 +272,9 @@ def test_tiled_iterations_match_gathered_ones(walls, lanes):
 
 
 def test_tiles_are_built_once_the_iterations_pay_for_them():
-    # At 120,384 particles tiles pay from 20 iterations on one list; the
-    # last solves' counts are 3 for a new handle.
+    # At 120,384 particles tiles pay from 20 iterations on one list. The
+    # last solves' counts are 3 for a new handle, so they are built once the
+    # lists have seen 40.
     x = scenes.lattice_block((76, 44, 36), 0.05, (0.1, 0.1, 0.1), jitter=0.001, seed=1)
     g = capi.TimeStepDFSPH(default_params(boundary_handling_method=BOUNDARY_NONE))
     g.set_fluid(x)
@@ -283,7 +284,7 @@ def test_tiles_are_built_once_the_iterations_pay_for_them():
         g.stage("densities")
         g.stage("dfsph_factor")
         g.stage("pressure_setup")
-        for _ in range(20):
+        for _ in range(40):
             g.stage("pressure_iter")
         assert "tile_lists" not in g.kernel_stats()
     g.stage("pressure_iter")

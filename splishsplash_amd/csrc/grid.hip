@@ -850,7 +850,10 @@ void build_lists_colmajor(hipStream_t s, const float4 *q, unsigned nq, const flo
 // (K = 225) 290 / 522 us, 100k uniform (K = 33) 235 / 212 us and clustered
 // (K = 260) 434 / 778 us, 131k uniform (K = 12) 258 / 181 us, 524k uniform
 // (K = 34) 698 / 438 us: few lanes per SIMD leave the memory latency open,
-// and a wave per query issues about four times the instructions.
+// and a wave per query issues about four times the instructions. The line is
+// that of even clouds. Long lists would keep the wave ahead beyond it (150k
+// clustered, K = 168: 484 / 780 us; 500k, K = 181: 1288 / 1600), but before
+// the first pass nothing tells them.
 constexpr unsigned CSR_WAVE_MAX = 1u << 17;
 // Queries of one launch with a wave each, of the `left` that remain: a launch
 // holds fewer than 2^32 threads. (Waves that take several queries in turn are

@@ -271,6 +271,40 @@ def test_tiled_iterations_match_gathered_ones(walls, lanes):
         assert ca[c] == cb[c], c
 
 
+@pytest.mark.parametrize("mode", ["reference", "previous"])
+def test_tiled_steps_match_gathered_ones_from_either_start(mode):
+    # Whole steps from both starts, from tiles and, with 300 fixed particles
+    # in one spot outside the walls whose row of candidates leaves no packed
+    # lists, gathered: with one lane per particle the fluid's sums are the
+    # same. Fixed iteration counts and time step: the spot has a share in the
+    # mean errors, and nothing else.
+    block = scenes.lattice_block((53, 50, 50), 0.05, (0.1, 0.1, 0.1), jitter=0.001, seed=1)
+    spot = np.float32([3.2, 2.6, 4.2]) + np.random.default_rng(8).uniform(-0.01, 0.01, (300, 3)).astype(np.float32)
+    params = default_params(cfl_method=0, time_step_size=0.001, min_iterations=24, max_iterations=24,
+                            max_iterations_v=8, max_error_v=1e-9, xsph=0.01)
+    v = perturbed_state(block, seed=11)[0]
+    out = []
+    for extra in (spot[:0], spot):
+        g = capi.TimeStepDFSPH(params)
+        g.set_fluid(scenes.f32(np.concatenate([block, extra])), scenes.f32(np.concatenate([v, 0 * extra])))
+        g.add_boundary_particles(scenes.box_wall_particles((0.0, 0.0, 0.0), (4.0, 3.0, 2.7), 0.05))
+        g.set_lanes_per_particle(1)
+        g.enable_timing()
+        g.init()
+        for solver in learned.SOLVERS:
+            g.set_warm_start_mode(solver, mode)
+            g.set_warm_start_policy(solver, 0)
+        g.set("state", np.concatenate([np.zeros(len(block)), np.full(len(extra), 2)]).astype(np.uint32))
+        g.step(4)
+        c = g.counters()
+        assert ("tile_lists" in g.kernel_stats()) == (len(extra) == 0) == (c["packed_lists"] == 1)
+        assert c["total_iterations"] == 4 * 24 and c["total_iterations_v"] == 4 * 8
+        out.append({f: g.get(f)[:len(block)] for f in ("position", "velocity", "p / rho^2", "p_v / rho^2")})
+    for f, a in out[0].items():
+        assert np.isfinite(a).all()
+        np.testing.assert_array_equal(a, out[1][f], err_msg=f)
+
+
 def test_tiles_are_built_once_the_iterations_pay_for_them():
     # At 120,384 particles tiles pay from 20 iterations on one list. The
     # last solves' counts are 3 for a new handle, so they are built once the
